@@ -152,13 +152,28 @@ struct KvItem {
   int b, kvh, k0t;  // sequence, KV head, first key of the tile
   SeqExt e;
   int qb_lo, nqb;   // first query block that sees the tile; blocks per head
+  // SPLIT: the chunk of the item's group * nqb blocks that this one is:
+  // chunk s of nc, at most len blocks each, its partials in slot.
+  int s, nc, len, slot;
 };
 
-// Position in a workgroup's program: item (round r), head hi, block qi.
+// Position in a workgroup's program: item (round r), head hi, block qi of
+// the head's segment.  Without SPLIT a segment is all nqb blocks of a head;
+// with it the chunk's part of them: segn blocks from block seg0 on, and
+// `left` blocks of the chunk after it.
+template <bool SPLIT>
 struct KvCursor {
   int r, hi, qi;
   bool done;
   KvItem it;
+  int seg0, segn, left;
+  __device__ __forceinline__ int block() const {  // query block of the sequence
+    return SPLIT ? it.qb_lo + seg0 + qi : it.qb_lo + qi;
+  }
+  __device__ __forceinline__ int seg_blocks() const { return SPLIT ? segn : it.nqb; }
+  __device__ __forceinline__ bool last_head(int group) const {
+    return SPLIT ? left == 0 : hi + 1 == group;
+  }
 };
 
 // One role's share of the ring DMA: the tiles in MASK of a block, wave w of
@@ -190,7 +205,8 @@ struct RingDma {
     drb = (uint32_t)P.delta.ss * 4u;
     loff = (uint32_t)lane * (is_delta ? drb : lrb);
   }
-  __device__ __forceinline__ void setup(const BwdParams& P, const KvCursor& c) {
+  template <bool SPLIT>
+  __device__ __forceinline__ void setup(const BwdParams& P, const KvCursor<SPLIT>& c) {
     // Past the last block the ring's last DMAs read nothing (zero-size
     // descriptors); no branch, so that every descriptor stays in registers.
     const Problem& p = P.p;
@@ -215,8 +231,9 @@ struct RingDma {
     }
   }
   // Exactly C::nb_of(MASK) VMEM instructions, unconditionally.
-  __device__ __forceinline__ void issue(const KvCursor& c, uint8_t* st, int w) const {
-    const uint32_t q0 = c.done ? 0u : (uint32_t)((c.it.qb_lo + c.qi) * C::BM);
+  template <bool SPLIT>
+  __device__ __forceinline__ void issue(const KvCursor<SPLIT>& c, uint8_t* st, int w) const {
+    const uint32_t q0 = c.done ? 0u : (uint32_t)(c.block() * C::BM);
     if constexpr ((MASK & kTileQ) != 0) dmq.issue_fixed(sq, st, w, q0 * qrb);
     if constexpr ((MASK & kTileR) != 0 && RPL > 0) dmr.issue_fixed(sr, st + C::QB, w, q0 * srb);
     if constexpr ((MASK & kTileO) != 0) dmo.issue_fixed(so, st + C::QB + C::RB, w, q0 * orb);
@@ -226,9 +243,10 @@ struct RingDma {
   }
 };
 
-template <int D, int RPL, bool F16, int RS>
+template <int D, int RPL, bool F16, int RS, bool SPLIT>
 __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
   using C = KvCfg<D, RPL, F16, RS>;
+  using Cursor = KvCursor<SPLIT>;
   __shared__ __attribute__((aligned(1024))) uint8_t st0[C::STAGE];
   __shared__ __attribute__((aligned(1024))) uint8_t st1[C::STAGE];
   __shared__ __attribute__((aligned(1024))) uint8_t st2[C::STAGE];
@@ -245,13 +263,24 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
   // this lane's key within the item in the wave's slice j
   auto krow_of = [&](int j) { return (kw * C::KPW + j) * 32 + l32; };
   const int G = gridDim.x, g = blockIdx.x;
-  const int n_items =
-      (P.tiles_k ? min(uni(*const_space(P.n_tiles_k)), P.k_tiles) : p.nseq * cdiv(p.sk, C::BN)) *
-      p.H_KV;
+  const int n_tiles =
+      P.tiles_k ? min(uni(*const_space(P.n_tiles_k)), P.k_tiles) : p.nseq * cdiv(p.sk, C::BN);
+  // SPLIT: the first split_tiles tiles of the list come as 2^split_log2
+  // chunks per KV head (some of them empty), the others whole.
+  const int n_cut = SPLIT ? min(n_tiles, P.split_tiles) : 0;
+  const int n_chunks = SPLIT ? (n_cut * p.H_KV) << P.split_log2 : 0;
+  const int n_items = n_chunks + (n_tiles - n_cut) * p.H_KV;
 
   auto decode = [&](int r) {
     KvItem x;
-    const int w = r * G + ((r & 1) ? G - 1 - g : g);
+    int w = r * G + ((r & 1) ? G - 1 - g : g);
+    bool cut = false;
+    if constexpr (SPLIT) {
+      cut = w < n_chunks;
+      x.s = cut ? w & ((1 << P.split_log2) - 1) : 0;
+      x.slot = w;
+      w = cut ? w >> P.split_log2 : w - n_chunks + n_cut * p.H_KV;
+    }
     const int tix = w / p.H_KV;
     x.kvh = w - tix * p.H_KV;
     int kt;
@@ -265,7 +294,22 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
     x.k0t = kt * C::BN;
     x.qb_lo = p.causal ? x.k0t / C::BM : 0;
     x.nqb = max(cdiv(x.e.lq, C::BM) - x.qb_lo, 0);
+    if constexpr (SPLIT) {
+      const KvChunks k = kv_chunks(p.group * x.nqb, cut ? P.split_log2 : 0);
+      x.nc = k.n;
+      x.len = k.len;
+    }
     return x;
+  };
+  // Enter the segment of head c.hi at block `from`, `blocks` blocks of the
+  // chunk to go.
+  auto enter = [&](Cursor& c, int from, int blocks) {
+    c.qi = 0;
+    if constexpr (SPLIT) {
+      c.seg0 = from;
+      c.segn = min(c.it.nqb - from, blocks);
+      c.left = blocks - c.segn;
+    }
   };
   auto round_valid = [&](int r) { return r * G + ((r & 1) ? G - 1 - g : g) < n_items; };
 
@@ -273,7 +317,7 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
   // 32-query blocks.  An item no query block can see (keys past every query
   // under the causal mask, or an empty query range) has zero gradients;
   // on_zero is called as the cursor passes it.
-  auto next_item = [&](KvCursor& c, auto&& on_zero) {
+  auto next_item = [&](Cursor& c, auto&& on_zero) {
     for (;;) {
       ++c.r;
       if (!round_valid(c.r)) {
@@ -283,32 +327,50 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
       c.it = decode(c.r);
       c.hi = 0;
       c.qi = 0;
-      if (c.it.nqb > 0) return;
+      if constexpr (SPLIT) {
+        if (c.it.s >= max(c.it.nc, 1)) continue;  // no such chunk
+      }
+      if (c.it.nqb > 0) {
+        if constexpr (SPLIT) {
+          const int first = c.it.s * c.it.len;
+          c.hi = first / c.it.nqb;
+          enter(c, first - c.hi * c.it.nqb, min(p.group * c.it.nqb - first, c.it.len));
+        }
+        return;
+      }
       on_zero(c.it);
     }
   };
-  auto advance = [&](KvCursor& c, auto&& on_zero) {
-    if (++c.qi < c.it.nqb) return;
+  auto advance = [&](Cursor& c, auto&& on_zero) {
+    if (++c.qi < c.seg_blocks()) return;
     c.qi = 0;
-    if (++c.hi < p.group) return;
+    if constexpr (SPLIT) {
+      if (c.left > 0) {
+        ++c.hi;
+        enter(c, 0, c.left);
+        return;
+      }
+    } else {
+      if (++c.hi < p.group) return;
+    }
     next_item(c, on_zero);
   };
-  auto start = [&](KvCursor& c, auto&& on_zero) {
+  auto start = [&](Cursor& c, auto&& on_zero) {
     c.r = -1;
     c.done = false;
     next_item(c, on_zero);
   };
   auto no_zero = [](const KvItem&) {};
   // The first block of the (item, head) after the cursor's (lookahead only).
-  auto next_seg = [&](KvCursor c) {
-    c.qi = 0;
-    if (++c.hi >= p.group) next_item(c, no_zero);
+  auto next_seg = [&](Cursor c) {
+    c.qi = c.seg_blocks() - 1;
+    advance(c, no_zero);
     return c;
   };
   // Whether this wave's keys meet block qi of the cursor's item.
-  auto block_active = [&](const KvCursor& c) {
+  auto block_active = [&](const Cursor& c) {
     const int wk0 = c.it.k0t + kw * 32 * C::KPW;
-    const int qbase = (c.it.qb_lo + c.qi) * C::BM;
+    const int qbase = c.block() * C::BM;
     return wk0 < c.it.e.lk && (!p.causal || qbase + C::BM - 1 >= wk0);
   };
 
@@ -415,7 +477,7 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
     // b = graph_scale[h] / c of the producer's current head (0 for a vanilla
     // head), set when the cursor enters a head.
     float bhp = 0.f;
-    auto head_scale = [&](const KvCursor& c) {
+    auto head_scale = [&](const Cursor& c) {
       const int h = c.it.kvh * p.group + c.hi;
       return uni_f(h < p.H_G ? *const_space(params_here()->gs + h) / p.c : 0.f);
     };
@@ -426,7 +488,7 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
     // rows 8 gq + 4 hl .. +3, gq = 0..3: -LSE in lsr[gq], delta in
     // lsr[4 + gq]), read after the rank MFMAs so that their latency hides
     // under the S chain.
-    auto scores = [&](const KvCursor& c, const uint8_t* cur, f32x16 (&sacc)[C::KPW],
+    auto scores = [&](const Cursor& c, const uint8_t* cur, f32x16 (&sacc)[C::KPW],
                       f32x16 (&dpacc)[C::KPW], f32x4_t (&lsr)[8]) {
       // (A vanilla head, or rank padding, has zero rank operands: its rank
       // MFMAs add exact zeros and keep the block one basic block.)
@@ -505,10 +567,10 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
     // of the consumer's MFMAs: for k-half j (query rows 16j..16j+15), lane
     // (key l32, half hl) holds rows 16j + 8i + 4hl + e, i = 0..1, e = 0..3,
     // i.e. accumulator registers 8j..8j+7.
-    auto softmax = [&](const KvCursor& c, uint8_t* pd, const f32x16 (&sacc_)[C::KPW],
+    auto softmax = [&](const Cursor& c, uint8_t* pd, const f32x16 (&sacc_)[C::KPW],
                        const f32x16 (&dpacc_)[C::KPW], const f32x4_t (&lsr)[8]) {
       const KvItem& x = c.it;
-      const int qbase = (x.qb_lo + c.qi) * C::BM;
+      const int qbase = c.block() * C::BM;
 #pragma unroll
       for (int ks = 0; ks < C::KPW; ++ks) {
       const f32x16& sacc = sacc_[ks];
@@ -574,9 +636,9 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
     // compiler adds no wait of its own.
     RingDma<C, RPL, kTileAll & ~C::CDMA> ring;
     ring.init(P, wv, lane);
-    KvCursor pc;  // the block being produced
+    Cursor pc;  // the block being produced
     start(pc, no_zero);
-    KvCursor ic = pc;  // the block whose tiles are issued next (two ahead)
+    Cursor ic = pc;  // the block whose tiles are issued next (two ahead)
     auto issue = [&](uint8_t* st) {
       if constexpr (C::NBP > 0) {
         ring.issue(ic, st, wv);
@@ -610,7 +672,7 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
         sign_k();
         bhp = head_scale(pc);
       }
-      KvCursor nx = pc;
+      Cursor nx = pc;
       advance(nx, no_zero);
       const bool act = block_active(pc);
       f32x16 sacc[C::KPW], dpacc[C::KPW];
@@ -624,7 +686,7 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
         // loaded here.
         // (One load site for each: branches around in-place loads of the
         // same registers made the compiler move them while in flight.)
-        const bool from_lds = C::KR && pc.it.nqb >= 2;
+        const bool from_lds = C::KR && pc.seg_blocks() >= 2;
         load_k(nx.it, nx.it.kvh * p.group + nx.hi, from_lds);
         load_v(nx.it);
         kr_in = from_lds;
@@ -725,7 +787,46 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
           for (int u = 0; u < 2; ++u) *(u32x4*)(rp + 32 * t + 16 * u) = w[t][u];
       }
     };
+    // SPLIT: a wave's fp32 accumulator tile (32 features x 32 keys) as it
+    // lies in the registers, 16 bytes per lane: tile `t` of the slice's
+    // part_tiles(D) (dK, then dV) in the chunk's slot, or of its RPL / 32 in
+    // a dRk slot.
+    auto put_tile = [&](float* base, const f32x16& a) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *(f32x4_t*)(base + i * 256 + lane * 4) =
+            f32x4_t{a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]};
+    };
+    auto part_rows = [&](const KvItem& x, int j, const f32x16* acc, int t0) {
+      float* base = params_here()->kv_part +
+                    ((int64_t)x.slot * (C::BN / 32) + kw * C::KPW + j) * (2 * C::NDB * 1024);
+#pragma unroll
+      for (int t = 0; t < C::NDB; ++t) put_tile(base + (t0 + t) * 1024, acc[t]);
+    };
+    auto part_drk = [&](const KvItem& x, int hi) {
+      if constexpr (SPLIT && C::NRB > 0) {
+        if (x.kvh * p.group + hi < p.H_G) {
+          const ParamsPtr pp = params_here();
+          const int64_t item = x.slot >> pp->split_log2;
+          const int64_t slot =
+              item * drk_slots(p.group, pp->split_log2) + x.s + hi;
+          static_for<C::KPW>([&](auto jj) {
+            constexpr int j = decltype(jj)::value;
+            float* base =
+                pp->drk_part + (slot * (C::BN / 32) + kw * C::KPW + j) * (C::NRB * 1024);
+#pragma unroll
+            for (int f = 0; f < C::NRB; ++f) put_tile(base + f * 1024, dkacc[j][C::NDB + f]);
+          });
+        }
+      }
+    };
     auto write_dk = [&](const KvItem& x, bool zero) {
+      if constexpr (SPLIT) {
+        if (x.nc > 1) {
+          static_for<C::KPW>([&](auto jj) { part_rows(x, decltype(jj)::value, dkacc[jj], 0); });
+          return;
+        }
+      }
       const ParamsPtr pp = params_here();
       static_for<C::KPW>([&](auto jj) {
         constexpr int j = decltype(jj)::value;
@@ -733,6 +834,12 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
       });
     };
     auto write_dv = [&](const KvItem& x, bool zero) {
+      if constexpr (SPLIT) {
+        if (x.nc > 1) {
+          static_for<C::KPW>([&](auto jj) { part_rows(x, decltype(jj)::value, dvacc[jj], C::NDB); });
+          return;
+        }
+      }
       const ParamsPtr pp = params_here();
       static_for<C::KPW>([&](auto jj) {
         constexpr int j = decltype(jj)::value;
@@ -784,7 +891,7 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
     // the producers switch to it.
     RingDma<C, RPL, C::CDMA> ring;
     ring.init(P, kw, lane);
-    KvCursor ic;  // the block whose tiles are issued next
+    Cursor ic;  // the block whose tiles are issued next
     auto issue = [&](uint8_t* st) {
       if constexpr (C::NBC > 0) {
         ring.issue(ic, st, kw);
@@ -900,7 +1007,7 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
     // first block.
     if (g == G - 1 && p.H_G > 0) reduce_dgs_waves(P, kw, C::NP, lane);
 
-    KvCursor cc;  // the block being consumed
+    Cursor cc;  // the block being consumed
     start(cc, on_zero);
     // Step t consumes block t - 1 (nothing at t = 0).  The barrier does not
     // wait for the consumers' own stores.
@@ -928,7 +1035,7 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
         // The producers switch to the next (item, head) at this step and
         // read its K | Rk from LDS after the barrier: this wave's DMA of it
         // must be complete.
-        if (kr_issued && !first && !cc.done && cc.qi + 1 == cc.it.nqb) {
+        if (kr_issued && !first && !cc.done && cc.qi + 1 == cc.seg_blocks()) {
           __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
           kr_issued = false;
         }
@@ -938,8 +1045,8 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
         // At the first block of an (item, head) of two or more blocks (the
         // producers read its K | Rk before this step's barrier); the
         // producers read the next one after the next barrier at the earliest.
-        if (!first && !cc.done && cc.qi == 0 && cc.it.nqb >= 2) {
-          const KvCursor ny = next_seg(cc);
+        if (!first && !cc.done && cc.qi == 0 && cc.seg_blocks() >= 2) {
+          const Cursor ny = next_seg(cc);
           if (!ny.done) {
             issue_kr(ny.it, ny.it.kvh * p.group + ny.hi);
             kr_issued = true;
@@ -954,14 +1061,17 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
       flush_dv();
       if (cc.done) return;
       if (block_active(cc)) consume(cur, pd);
-      if (cc.qi + 1 < cc.it.nqb) {
+      if (cc.qi + 1 < cc.seg_blocks()) {
         ++cc.qi;
         return;
       }
       __builtin_amdgcn_sched_barrier(0);
       const KvItem x = cc.it;
-      const bool last_head = cc.hi + 1 == p.group;
-      write_drk(x, x.kvh * p.group + cc.hi, false);
+      const bool last_head = cc.last_head(p.group);
+      if (SPLIT && cc.segn != x.nqb)
+        part_drk(x, cc.hi);
+      else
+        write_drk(x, x.kvh * p.group + cc.hi, false);
       if (last_head) {
         write_dk(x, false);
         dv_pending = true;
@@ -998,15 +1108,19 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
 
 // One non-template kernel per (D, rank, element type) so that each has a
 // host stub.  Rank names: 0, 32 and 64 are the padded rank tiles; 16 is the
-// 32-wide tile with one rank step (R <= 16).
-#define FNA2_DKDV_KERNEL(D, RNAME, RPL, RS)                                              \
-  __global__ __launch_bounds__(512, 1) void dkdv_kernel_d##D##_r##RNAME(const BwdParams P) { \
-    dkdv_body<D, RPL, false, RS>(P);                                                     \
-  }                                                                                      \
-  __global__ __launch_bounds__(512, 1) void dkdv_kernel_d##D##_r##RNAME##_f16(             \
-      const BwdParams P) {                                                               \
-    dkdv_body<D, RPL, true, RS>(P);                                                      \
+// 32-wide tile with one rank step (R <= 16).  _split: the items of the first
+// tiles in chunks, kept apart from the kernels without (the scalar state of
+// a chunk costs the step loop); R <= 16 takes two rank steps there.
+#define FNA2_DKDV_ONE(NAME, D, RPL, F16, RS, SPLIT)                   \
+  __global__ __launch_bounds__(512, 1) void NAME(const BwdParams P) { \
+    dkdv_body<D, RPL, F16, RS, SPLIT>(P);                             \
   }
+#define FNA2_DKDV_KERNEL(D, RNAME, RPL, RS)                            \
+  FNA2_DKDV_ONE(dkdv_kernel_d##D##_r##RNAME, D, RPL, false, RS, false) \
+  FNA2_DKDV_ONE(dkdv_kernel_d##D##_r##RNAME##_f16, D, RPL, true, RS, false)
+#define FNA2_DKDV_SPLIT(D, RPL)                                                   \
+  FNA2_DKDV_ONE(dkdv_kernel_d##D##_r##RPL##_split, D, RPL, false, RPL / 16, true) \
+  FNA2_DKDV_ONE(dkdv_kernel_d##D##_r##RPL##_f16_split, D, RPL, true, RPL / 16, true)
 FNA2_DKDV_KERNEL(64, 0, 0, 0)
 FNA2_DKDV_KERNEL(64, 16, 32, 1)
 FNA2_DKDV_KERNEL(64, 32, 32, 2)
@@ -1015,7 +1129,15 @@ FNA2_DKDV_KERNEL(128, 0, 0, 0)
 FNA2_DKDV_KERNEL(128, 16, 32, 1)
 FNA2_DKDV_KERNEL(128, 32, 32, 2)
 FNA2_DKDV_KERNEL(128, 64, 64, 4)
+FNA2_DKDV_SPLIT(64, 0)
+FNA2_DKDV_SPLIT(64, 32)
+FNA2_DKDV_SPLIT(64, 64)
+FNA2_DKDV_SPLIT(128, 0)
+FNA2_DKDV_SPLIT(128, 32)
+FNA2_DKDV_SPLIT(128, 64)
+#undef FNA2_DKDV_SPLIT
 #undef FNA2_DKDV_KERNEL
+#undef FNA2_DKDV_ONE
 
 }  // namespace
 
@@ -1023,23 +1145,29 @@ hipError_t launch_bwd_dkdv(const BwdParams& P, int rpl, int grid, hipStream_t s)
   if (grid <= 0) return hipSuccess;
   void (*k)(const BwdParams) = nullptr;
   const bool r16 = rpl == 32 && P.p.R <= 16;  // one rank step
-  if (P.p.f16) {
-    if (P.p.D == 64)
-      k = rpl == 0 ? dkdv_kernel_d64_r0_f16
-          : rpl == 32 ? (r16 ? dkdv_kernel_d64_r16_f16 : dkdv_kernel_d64_r32_f16)
-                      : dkdv_kernel_d64_r64_f16;
-    if (P.p.D == 128)
-      k = rpl == 0 ? dkdv_kernel_d128_r0_f16
-          : rpl == 32 ? (r16 ? dkdv_kernel_d128_r16_f16 : dkdv_kernel_d128_r32_f16)
-                      : dkdv_kernel_d128_r64_f16;
-  } else {
-    if (P.p.D == 64)
-      k = rpl == 0 ? dkdv_kernel_d64_r0
-          : rpl == 32 ? (r16 ? dkdv_kernel_d64_r16 : dkdv_kernel_d64_r32) : dkdv_kernel_d64_r64;
-    if (P.p.D == 128)
-      k = rpl == 0 ? dkdv_kernel_d128_r0
-          : rpl == 32 ? (r16 ? dkdv_kernel_d128_r16 : dkdv_kernel_d128_r32) : dkdv_kernel_d128_r64;
+  const bool f16 = P.p.f16 != 0, split = P.split_tiles > 0;
+#define FNA2_DKDV_OF(D, RNAME) (f16 ? dkdv_kernel_d##D##_r##RNAME##_f16 : dkdv_kernel_d##D##_r##RNAME)
+#define FNA2_DKDV_SPLIT_OF(D, RPL) \
+  (f16 ? dkdv_kernel_d##D##_r##RPL##_f16_split : dkdv_kernel_d##D##_r##RPL##_split)
+  if (P.p.D == 64) {
+    if (split)
+      k = rpl == 0 ? FNA2_DKDV_SPLIT_OF(64, 0)
+          : rpl == 32 ? FNA2_DKDV_SPLIT_OF(64, 32) : FNA2_DKDV_SPLIT_OF(64, 64);
+    else
+      k = rpl == 0 ? FNA2_DKDV_OF(64, 0)
+          : rpl == 32 ? (r16 ? FNA2_DKDV_OF(64, 16) : FNA2_DKDV_OF(64, 32)) : FNA2_DKDV_OF(64, 64);
   }
+  if (P.p.D == 128) {
+    if (split)
+      k = rpl == 0 ? FNA2_DKDV_SPLIT_OF(128, 0)
+          : rpl == 32 ? FNA2_DKDV_SPLIT_OF(128, 32) : FNA2_DKDV_SPLIT_OF(128, 64);
+    else
+      k = rpl == 0 ? FNA2_DKDV_OF(128, 0)
+          : rpl == 32 ? (r16 ? FNA2_DKDV_OF(128, 16) : FNA2_DKDV_OF(128, 32))
+                      : FNA2_DKDV_OF(128, 64);
+  }
+#undef FNA2_DKDV_SPLIT_OF
+#undef FNA2_DKDV_OF
   if (!k || (rpl != 0 && rpl != 32 && rpl != 64)) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k, dim3(grid), dim3(512), 0, s, P);
   return hipGetLastError();

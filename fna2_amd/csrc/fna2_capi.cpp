@@ -161,6 +161,92 @@ BwdWs bwd_ws(const fna2_problem& p) {
   return w;
 }
 
+// dK/dV items in chunks.  The persistent dK/dV kernel deals (key tile, KV
+// head) items to the CUs; where these are fewer than the CUs, or one item is
+// longer than a CU's share of the work, the time is the longest item's.
+// Then the items of the first `tiles` tiles of the list (longest first) run
+// in up to 2^log2 chunks of their (query head, query block) sequence, which
+// write fp32 partials to the workspace for a reduction kernel.  The rule
+// compares, in blocks (32 queries against a key tile), the longest chunk and
+// a CU's share with what entering a chunk costs (kEnter) and the reduction
+// (its launch and the partials written and read); in varlen mode, where the
+// host does not know the lengths, it takes the pack as total_k / max_seqlen
+// sequences of the hinted length.
+//
+// Measured (dK/dV and its reduction, us, whole items -> the rule's chunks):
+// B2 H16/4 L1531 d128 fp16 238 -> 88 (chunks of 1/2: 138, 1/4: 86, 1/8: 96,
+// 1/16: 120), B1 H8/4 L512 d64 51 -> 24, B1 H32/8 L1024 d128 158 -> 60, B1
+// H8/4 L8192 d128 580 -> 355.  Where the rule keeps them whole: B1 H16 L2048
+// d128 (256 items) 85 whole, 82 in halves, 104 in quarters; B1 H8 L128 15
+// against 18.
+struct KvSplit {
+  int log2 = 0;
+  int64_t tiles = 0;
+  size_t kv_part = 0, drk_part = 0, bytes = 0;  // offsets in the split's own region
+};
+constexpr int kSplitCUs = 256;  // (a fixed figure: the size depends on the arguments alone)
+constexpr int64_t kSplitMaxBytes = (int64_t)512 << 20;
+
+KvSplit kv_split(const fna2_problem& p) {
+  KvSplit best;
+  const Grids g = grids(p);
+  if (p.batch <= 0 || g.kv_grid <= 0) return best;
+  const int bn = kv_tile(p);
+  const int group = p.heads / p.heads_kv;
+  int64_t lq, lk, nseq;
+  if (p.varlen) {
+    lk = p.seqlen_k > 0 && p.seqlen_k < p.total_k ? p.seqlen_k : p.total_k;
+    lq = p.seqlen_q > 0 && p.seqlen_q < p.total_q ? p.seqlen_q : p.total_q;
+    nseq = lk > 0 ? std::max<int64_t>(p.total_k / lk, 1) : 1;
+  } else {
+    lk = p.seqlen_k;
+    lq = p.seqlen_q;
+    nseq = p.batch;
+  }
+  const int64_t qb = cdiv64(lq, kKvBM), kt = cdiv64(lk, bn), lo = p.causal ? bn / kKvBM : 0;
+  if (qb <= 0 || kt <= 0) return best;
+  // blocks of one sequence and head: sum over its key tiles of qb - lo t
+  const int64_t seen = lo > 0 ? std::min<int64_t>(kt, cdiv64(qb, lo)) : kt;
+  const int64_t per_head = seen * qb - lo * (seen * (seen - 1) / 2);
+  const int64_t items = nseq * kt * p.heads_kv;
+  const int64_t total = nseq * p.heads * per_head;
+  const int64_t longest = (int64_t)group * qb;
+  const int64_t rpl = fna2::padded_rank32(p.heads_graph, p.rank);
+  const int64_t cut = p.varlen ? std::min<int64_t>(g.kv_tiles, cdiv64(p.total_k, bn) + 8)
+                               : g.kv_tiles;
+  constexpr double kEnter = 4, kLaunch = 5, kBytesPerBlock = 4e6;
+  auto cost = [&](int log2) {
+    const int64_t n = (int64_t)1 << log2;
+    const double len = (double)std::max<int64_t>(cdiv64(longest, n), log2 ? fna2::kKvMinChunk : 1);
+    const double chunks = std::min((double)items * n, std::max((double)total / fna2::kKvMinChunk,
+                                                               (double)items));
+    double t = std::max(len + kEnter, (total + kEnter * chunks) / kSplitCUs);
+    if (log2 > 0)
+      t += kLaunch + chunks * bn * (2 * p.head_dim + rpl) * 8.0 / kBytesPerBlock;
+    return t;
+  };
+  double least = 0.9 * cost(0);
+  for (int log2 = 1; log2 <= 4; ++log2) {
+    KvSplit s;
+    s.log2 = log2;
+    s.tiles = cut;
+    const int64_t kv = (int64_t)p.heads_kv * ((int64_t)1 << log2) * bn * 2 * p.head_dim * 4;
+    const int64_t dr = p.heads_graph > 0
+                           ? (int64_t)p.heads_kv * fna2::drk_slots(group, log2) * bn * rpl * 4
+                           : 0;
+    s.tiles = std::min<int64_t>(s.tiles, kSplitMaxBytes / (kv + dr));
+    if (s.tiles <= 0 || (s.tiles * p.heads_kv) << log2 > kMaxGrid) continue;
+    s.drk_part = align_up((size_t)(s.tiles * kv));
+    s.bytes = s.drk_part + align_up((size_t)(s.tiles * dr));
+    const double t = cost(log2);
+    if (t < least) {
+      least = t;
+      best = s;
+    }
+  }
+  return best;
+}
+
 // Plan (varlen): the query-tile list the forward and the dQ kernel share
 // (the same tile shape) and the dK/dV key-tile list.
 static_assert(kFwdBM == kDqBM && kFwdBN == kDqBN, "the forward and dQ share their tile list");
@@ -414,6 +500,11 @@ size_t fna2_bwd_workspace_bytes(const fna2_problem* p) {
   return bwd_ws(*p).bytes;
 }
 
+size_t fna2_bwd_split_bytes(const fna2_problem* p) {
+  if (!p || check_problem(*p) != FNA2_OK) return 0;
+  return kv_split(*p).bytes;
+}
+
 size_t fna2_plan_bytes(const fna2_problem* p) {
   if (!p || check_problem(*p) != FNA2_OK) return 0;
   return plan_layout(*p).bytes;
@@ -608,9 +699,25 @@ int fna2_bwd(const fna2_bwd_args* a, void* stream_ptr) {
     if (rows_q(p) > 0 && fna2::launch_bwd_dq(K, rpl, dq_grid, stream) != hipSuccess)
       return FNA2_E_LAUNCH;
     if (!mark(a->events, 1, stream) || !mark(a->events, 2, stream)) return FNA2_E_LAUNCH;
+    // Items in chunks, where the rule asks for it and the caller's workspace
+    // has the room (bwd_ws and fna2_bwd_split_bytes).
+    const KvSplit sp = kv_split(p);
+    int64_t items = g.kv_grid;
+    if (sp.bytes > 0 && rows_q(p) > 0 && a->workspace_bytes >= w.bytes + sp.bytes &&
+        aligned(a->workspace, 16)) {
+      char* base = (char*)a->workspace + w.bytes;
+      K.split_tiles = (int)sp.tiles;
+      K.split_log2 = sp.log2;
+      K.kv_part = (float*)(base + sp.kv_part);
+      K.drk_part = (float*)(base + sp.drk_part);
+      items += ((sp.tiles * p.heads_kv) << sp.log2) - sp.tiles * p.heads_kv;
+    }
     // persistent: one workgroup per CU walks the (key tile, KV head) items
-    const int kv_grid = (int)std::min<int64_t>(g.kv_grid, n_cu);
+    const int kv_grid = (int)std::min<int64_t>(items, n_cu);
     if (rows_k(p) > 0 && fna2::launch_bwd_dkdv(K, rpl, kv_grid, stream) != hipSuccess)
+      return FNA2_E_LAUNCH;
+    if (K.split_tiles > 0 && rows_k(p) > 0 &&
+        fna2::launch_bwd_kv_reduce(K, rpl, stream) != hipSuccess)
       return FNA2_E_LAUNCH;
     if (!mark(a->events, 3, stream)) return FNA2_E_LAUNCH;
   } else if (p.varlen && p.batch == 0 && (rows_q(p) > 0 || rows_k(p) > 0)) {

@@ -27,6 +27,11 @@ struct BwdParams {
   const int* n_tiles_q;
   const TileRec* tiles_k;  // varlen: key tiles (dK/dV kernel)
   const int* n_tiles_k;
+  // dK/dV items in chunks (split_tiles > 0): the first split_tiles key tiles
+  // of the list, per KV head, in up to 2^split_log2 chunks of their blocks.
+  int split_tiles, split_log2;
+  float* kv_part;   // [split_tiles][H_KV][2^split_log2] slots of dK | dV
+  float* drk_part;  // [split_tiles][H_KV][drk_slots] slots of dRk
   int zero_uncovered;  // varlen: the dQ kernel's spare workgroups zero the
                        // gradient rows of tokens outside every sequence
 };
@@ -46,6 +51,25 @@ constexpr int kFwdBN = 64;
 constexpr int kv_kpw(int D, int rpl) { return (D == 64 && rpl <= 32) ? 2 : 1; }
 constexpr int kv_bn(int D, int rpl) { return 128 * kv_kpw(D, rpl); }
 constexpr int kKvBM = 32;
+
+// A dK/dV item of `blocks` (head, query block) pairs in up to 2^log2 chunks
+// of equal length, at least kKvMinChunk blocks each: a shorter one costs
+// more to enter and leave (row loads, partial stores) than it spreads.
+constexpr int kKvMinChunk = 4;
+struct KvChunks {
+  int n, len;
+};
+__host__ __device__ inline KvChunks kv_chunks(int blocks, int log2) {
+  KvChunks k;
+  k.len = (blocks + (1 << log2) - 1) >> log2;
+  if (k.len < kKvMinChunk) k.len = kKvMinChunk;
+  k.n = log2 > 0 ? (blocks + k.len - 1) / k.len : 1;
+  if (log2 <= 0) k.len = blocks;
+  return k;
+}
+// dRk partial slots of an item: head hi's part in chunk s goes to slot
+// s + hi (both only grow along the item's blocks).
+__host__ __device__ inline int drk_slots(int group, int log2) { return group + (1 << log2) - 1; }
 constexpr int kDqBM = 128;
 constexpr int kDqBN = 64;
 
@@ -109,6 +133,8 @@ hipError_t launch_decode_merge(const DecodeParams& P, hipStream_t s);
 hipError_t launch_fwd(const FwdParams& P, int rp, int grid, hipStream_t s);
 hipError_t launch_bwd_dkdv(const BwdParams& P, int rpl, int grid, hipStream_t s);
 hipError_t launch_bwd_dq(const BwdParams& P, int rpl, int grid, hipStream_t s);
+// Sums the chunks' partials into dK, dV and dRk (fixed order).
+hipError_t launch_bwd_kv_reduce(const BwdParams& P, int rpl, hipStream_t s);
 hipError_t launch_bwd_dgs(const BwdParams& P, hipStream_t s);
 
 // d_gs[h] = sum of the dQ kernel's partials of head h in a fixed order

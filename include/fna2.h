@@ -303,6 +303,11 @@ int fna2_check_bwd(const fna2_bwd_args* args);
 /* Workspace bytes the forward / backward need for this problem. */
 size_t fna2_fwd_workspace_bytes(const fna2_problem* p);
 size_t fna2_bwd_workspace_bytes(const fna2_problem* p);
+/* Optional: bytes that a fna2_bwd of this problem makes use of beyond
+ * fna2_bwd_workspace_bytes (0: none).  Given a workspace of the sum, it runs
+ * dK/dV items that would leave CUs idle in chunks (the same sums, fp32
+ * partials added in a fixed order); with less it runs them whole. */
+size_t fna2_bwd_split_bytes(const fna2_problem* p);
 
 /* Bytes of a plan (the varlen tile lists of the forward and the backward:
  * device-built, so no host synchronisation); 0 in dense mode.  No

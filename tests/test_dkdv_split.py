@@ -1,0 +1,173 @@
+"""dK/dV items in chunks (fna2_bwd_dkdv.hip with SPLIT, kv_reduce_kernel).
+
+CPU: the chunks of an item cover its (head, query block) sequence once, and
+the reduction reads exactly the dRk slots the chunks write (kv_chunks,
+drk_slots in fna2_kernels.h restated).  GPU: gradients of shapes whose items
+run in chunks against the oracle, and against the same call without the room
+for chunks (the whole-item kernels): chunks that end inside a head, at heads'
+ends, empty chunks, key tiles no query sees, ragged packs, cross lengths.
+"""
+import ctypes
+import math
+
+import pytest
+import torch
+
+from . import helpers as Hp
+
+MIN_CHUNK = 4
+
+
+def kv_chunks(blocks, log2):
+    n = max(-(-blocks // (1 << log2)), MIN_CHUNK)
+    return -(-blocks // n), n
+
+
+@pytest.mark.parametrize("log2", [1, 2, 3, 4])
+@pytest.mark.parametrize("group", [1, 2, 3, 8])
+def test_chunks_cover_an_item_once(group, log2):
+    for nqb in list(range(0, 40)) + [127, 512]:
+        n, length = kv_chunks(group * nqb, log2)
+        assert n <= 1 << log2
+        seen, wrote, whole = [], {}, set()
+        for s in range(n):  # the cursor's walk of a chunk
+            first = s * length
+            hi, at = divmod(first, nqb)
+            left = min(group * nqb - first, length)
+            while True:
+                seg = min(nqb - at, left)
+                assert seg > 0
+                left -= seg
+                seen += [(hi, at + i) for i in range(seg)]
+                if seg == nqb:
+                    whole.add(hi)
+                else:
+                    assert s + hi not in wrote, "two segments in one dRk slot"
+                    wrote[s + hi] = hi
+                    assert s + hi < group + (1 << log2) - 1
+                if left == 0:
+                    break
+                hi, at = hi + 1, 0
+        assert seen == [(h, q) for h in range(group) for q in range(nqb)]
+        reads = {}
+        for h in range(group if n > 1 else 0):  # kv_reduce_kernel
+            c0, c1 = h * nqb // length, ((h + 1) * nqb - 1) // length + 1
+            if c1 - c0 > 1:
+                reads.update({c + h: h for c in range(c0, c1)})
+                assert h not in whole
+            else:
+                assert h in whole
+        if n > 1:
+            assert reads == wrote
+        else:
+            assert not wrote
+
+
+def _split_bytes(prob):
+    from fna2_amd import _capi
+    return int(_capi.lib().fna2_bwd_split_bytes(ctypes.byref(prob)))
+
+
+def _problem(varlen, B, Sq, Sk, H, HKV, HG, D, R, causal, cu=None):
+    import importlib
+    F = importlib.import_module("fna2_amd.flash_naylis_attn")
+    tq, tk = (Sq, Sk) if varlen else (0, 0)
+    return F._problem(varlen, B, Sq, Sk, tq, tk, H, HKV, HG, D, R, causal, 0.1, cu, cu)
+
+
+def test_split_rule():
+    """Chunks where the items leave CUs idle, none where they fill them."""
+    few = _split_bytes(_problem(False, 2, 1531, 1531, 16, 4, 12, 128, 24, True))
+    assert few > 0
+    # fp32 dK | dV of every chunk of every 128-key tile, at least two chunks
+    assert few >= 2 * 2 * 12 * 4 * 2 * 128 * 2 * 128 * 4 // 2
+    assert _split_bytes(_problem(False, 4, 2048, 2048, 16, 16, 16, 64, 16, True)) == 0
+    assert _split_bytes(_problem(False, 1, 16384, 16384, 32, 32, 32, 128, 64, True)) == 0
+    assert _split_bytes(_problem(False, 1, 64, 64, 8, 8, 8, 64, 32, True)) == 0
+    assert _split_bytes(_problem(False, 2, 0, 128, 4, 4, 4, 64, 32, True)) == 0
+
+
+DENSE = [  # B, Sq, Sk, H, HKV, HG, D, R, causal, fp16
+    (1, 512, 512, 8, 4, 4, 64, 32, True, False),
+    (1, 1000, 1000, 3, 1, 2, 64, 16, True, False),
+    (1, 700, 700, 6, 2, 5, 64, 64, False, False),
+    (1, 900, 900, 4, 2, 3, 128, 64, True, False),
+    (2, 513, 513, 8, 2, 6, 128, 24, True, True),
+    (1, 1025, 1025, 2, 2, 1, 64, 8, True, True),
+    (1, 333, 1200, 4, 1, 4, 128, 32, True, False),   # key tiles no query sees
+    (1, 1500, 70, 4, 4, 4, 128, 0, False, False),    # one key tile, no rank
+]
+
+
+def _run_dense(gpu, c, split):
+    from fna2_amd import flash_naylis_attn as api
+    import importlib
+    F = importlib.import_module("fna2_amd.flash_naylis_attn")
+    B, Sq, Sk, H, HKV, HG, D, R, causal, fp16 = c
+    ins = Hp.make_dense(B, H, Sq, D, HKV, HG if R else 0, R, seed=Sq + D + R, Sk=Sk)
+    if fp16:
+        ins = tuple(t if t is None or i in (3, 4, 5) else t.half() for i, t in enumerate(ins))
+    q, k, v, rq, rk, gs, dout = (None if t is None else t.to(gpu) for t in ins)
+    scale = 1 / math.sqrt(D)
+    out, lse = F._fna2_forward(q, k, v, rq, rk, gs, scale, causal)
+    keep = F._capi.lib().fna2_bwd_split_bytes
+    try:
+        if not split:
+            F._capi.lib().fna2_bwd_split_bytes = lambda p: 0
+        grads = F._fna2_backward(dout, q, k, v, rq, rk, gs, out, lse, scale, causal)
+    finally:
+        F._capi.lib().fna2_bwd_split_bytes = keep
+    torch.cuda.synchronize()
+    return ins, scale, grads
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", DENSE, ids=lambda c: "-".join(map(str, c)))
+def test_dense_chunks(gpu, case):
+    B, Sq, Sk, H, HKV, HG, D, R, causal, fp16 = case
+    print(case, flush=True)
+    assert _split_bytes(_problem(False, B, Sq, Sk, H, HKV, HG if R else 0, D, R, causal)) > 0
+    ins, scale, got = _run_dense(gpu, case, True)
+    _, _, whole = _run_dense(gpu, case, False)
+    _, _, again = _run_dense(gpu, case, True)
+    for a, b, c in zip(got, whole, again):
+        if a is None:
+            continue
+        assert torch.equal(a, c), "not reproducible"
+        # the same fp32 terms in another order, rounded once to 16 bits
+        # (2^-9 of a value, half the values at most one step apart)
+        assert Hp.rel_norm(a, b.double().cpu().numpy()) < 4e-3
+    q, k, v, rq, rk, gs, dout = ins
+    _, _, ref = Hp.oracle_fwd_bwd(q, k, v, rq, rk, gs, dout, scale, causal)
+    Hp.check_grads(got[:5], ref[:5])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("D,R", [(64, 16), (128, 32)])
+def test_varlen_chunks(gpu, causal, D, R):
+    """One long sequence beside short and empty ones, tokens outside every
+    sequence, a vanilla head; the long tiles in chunks, the short ones whole."""
+    import importlib
+    F = importlib.import_module("fna2_amd.flash_naylis_attn")
+    lens, H, HKV, HG = [40, 0, 1300, 17, 129], 4, 2, 3
+    q, k, v, rq, rk, gs, dout, cu, _ = Hp.make_varlen(lens + [9], H, D, HKV, HG, R, seed=D)
+    cu = cu[:-1]
+    dev = [t.to(gpu) for t in (q, k, v, rq, rk, gs, dout, cu)]
+    dq, dk, dv, drq, drk, dgs, ddo, dcu = dev
+    scale = 1 / math.sqrt(D)
+    prob = F._problem(True, len(lens), 1300, 1300, q.shape[0], q.shape[0], H, HKV, HG, D, R,
+                      causal, scale, dcu, dcu)
+    assert _split_bytes(prob) > 0
+    print("varlen chunks", D, R, causal, flush=True)
+    out, lse = F._fna2_forward_varlen(dq, dk, dv, drq, drk, dgs, dcu, dcu, 1300, 1300, scale,
+                                      causal)
+    got = F._fna2_backward_varlen(ddo, dq, dk, dv, drq, drk, dgs, out, lse, dcu, dcu, 1300, 1300,
+                                  scale, causal)
+    torch.cuda.synchronize()
+    n = sum(lens)
+    ref_o, ref_l, ref = Hp.oracle_fwd_bwd(q, k, v, rq, rk, gs, dout, scale, causal, cu.numpy(),
+                                          cu.numpy())
+    for g, r in zip(got[:5], ref[:5]):
+        assert not g[n:].any(), "rows outside every sequence"
+        assert Hp.rel_norm(g[:n], r[:n]) < Hp.TOL_GRAD
