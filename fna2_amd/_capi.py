@@ -234,6 +234,26 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The torch binding (``csrc/fna2_torch.cpp``), bound to ``lib()``'s
+    functions.  Raises if it has not been built."""
+    global _native
+    if _native is None:
+        handle = lib()
+        from importlib import import_module
+        try:
+            mod = import_module("._torch_binding", __package__)
+        except ImportError as e:
+            raise RuntimeError("fna2_amd/_torch_binding.so does not load; build it with "
+                               f"`python -m fna2_amd.build` ({e})") from e
+        mod.bind({n: ctypes.cast(getattr(handle, n), ctypes.c_void_p).value for n in SIGNATURES})
+        _native = mod
+    return _native
+
+
 def available() -> bool:
     try:
         lib()

@@ -196,6 +196,29 @@ def _events(names):
     return _timer.take(names)
 
 
+def _native_fwd(q, k, v, r_q, r_k, graph_scale, scale, causal, cu_q=None, cu_k=None, max_q=0,
+                max_k=0, plan=None, plan_filled=False, head_major=False):
+    """(out, lse) by the native launch path, or None for the calls it leaves
+    to the Python launcher: layouts and dtypes to convert, empty tensors,
+    per-kernel timing, errors to raise."""
+    if _timer is not None or not q.is_cuda:
+        return None
+    return _capi.native().attn_fwd(q, k, v, r_q, r_k, graph_scale, scale, bool(causal), cu_q, cu_k,
+                                   max_q, max_k, plan, bool(plan_filled), head_major)
+
+
+def _native_bwd(dout, q, k, v, r_q, r_k, graph_scale, out, lse, scale, causal, cu_q=None,
+                cu_k=None, max_q=0, max_k=0, plan=None, grads_out=None):
+    """The backward's gradients by the native launch path, or None (as above)."""
+    if _timer is not None or not q.is_cuda:
+        return None
+    to = (None,) * 5 if grads_out is None else grads_out
+    if to[0] is not None or to[1] is not None:
+        return None
+    return _capi.native().attn_bwd(dout, q, k, v, r_q, r_k, graph_scale, out, lse, scale,
+                                   bool(causal), cu_q, cu_k, max_q, max_k, plan, *to[2:])
+
+
 def _workspace(fn, prob: _capi.Problem, dev) -> torch.Tensor:
     nbytes = int(fn(ctypes.byref(prob)))
     return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
@@ -257,6 +280,9 @@ def _fna2_forward(
     is_causal: bool,
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """Dense forward; returns (out, lse).  Mirrors FNA2/flash_naylis_attn.py:700-753."""
+    done = _native_fwd(q, k, v, r_q, r_k, graph_scale, softmax_scale, is_causal)
+    if done is not None:
+        return done
     B, H, S, D = q.shape
     H_KV, S_k = k.shape[1], k.shape[2]
     H_G = 0 if r_q is None else r_q.shape[1]
@@ -308,6 +334,10 @@ def _fna2_forward_varlen(
     ``plan_filled``: an earlier forward of this problem filled ``plan`` for
     these cu_seqlens, unchanged since: its lists are reused (no list-building
     launch)."""
+    done = _native_fwd(q, k, v, r_q, r_k, graph_scale, softmax_scale, is_causal, cu_seqlens_q,
+                       cu_seqlens_k, max_seqlen_q, max_seqlen_k, plan, plan_filled, lse_head_major)
+    if done is not None:
+        return done
     total_q, H, D = q.shape
     total_k, H_KV = k.shape[0], k.shape[1]
     H_G = 0 if r_q is None else r_q.shape[1]
@@ -356,6 +386,10 @@ def _fna2_backward(
 ) -> tuple:
     """Dense backward; returns (dq, dk, dv, dr_q, dr_k, d_gs).  Mirrors :807-892.
     ``grads_out``: as for ``_fna2_backward_varlen``."""
+    done = _native_bwd(dout, q, k, v, r_q, r_k, graph_scale, out, lse, softmax_scale, is_causal,
+                       grads_out=grads_out)
+    if done is not None:
+        return done
     B, H, S, D = q.shape
     H_KV, S_k = k.shape[1], k.shape[2]
     H_G = 0 if r_q is None else r_q.shape[1]
@@ -394,6 +428,10 @@ def _fna2_backward_varlen(
     ``plan``: the one the forward of the same problem filled (optional).
     ``grads_out``: (dq, dk, dv, dr_q, dr_k) tensors to write the gradients
     into, None entries allocated here (any row strides, unit last stride)."""
+    done = _native_bwd(dout, q, k, v, r_q, r_k, graph_scale, out, lse, softmax_scale, is_causal,
+                       cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, plan, grads_out)
+    if done is not None:
+        return done
     total_q, H, D = q.shape
     total_k, H_KV = k.shape[0], k.shape[1]
     H_G = 0 if r_q is None else r_q.shape[1]

@@ -100,7 +100,6 @@ DENSE = [  # B, Sq, Sk, H, HKV, HG, D, R, causal, fp16
 
 
 def _run_dense(gpu, c, split):
-    from fna2_amd import flash_naylis_attn as api
     import importlib
     F = importlib.import_module("fna2_amd.flash_naylis_attn")
     B, Sq, Sk, H, HKV, HG, D, R, causal, fp16 = c
@@ -110,13 +109,15 @@ def _run_dense(gpu, c, split):
     q, k, v, rq, rk, gs, dout = (None if t is None else t.to(gpu) for t in ins)
     scale = 1 / math.sqrt(D)
     out, lse = F._fna2_forward(q, k, v, rq, rk, gs, scale, causal)
-    keep = F._capi.lib().fna2_bwd_split_bytes
+    lib = F._capi.lib()
+    keep, native = lib.fna2_bwd_split_bytes, F._native_bwd
     try:
-        if not split:
-            F._capi.lib().fna2_bwd_split_bytes = lambda p: 0
+        if not split:  # the Python launcher, with a workspace that has no room for chunks
+            lib.fna2_bwd_split_bytes = lambda p: 0
+            F._native_bwd = lambda *a, **kw: None
         grads = F._fna2_backward(dout, q, k, v, rq, rk, gs, out, lse, scale, causal)
     finally:
-        F._capi.lib().fna2_bwd_split_bytes = keep
+        lib.fna2_bwd_split_bytes, F._native_bwd = keep, native
     torch.cuda.synchronize()
     return ins, scale, grads
 

@@ -1,0 +1,116 @@
+"""The native launch path (csrc/fna2_torch.cpp) against the Python launchers:
+the same call through both gives the same bits, and calls it does not take
+(layouts to copy, dtypes to convert, errors to raise) go on as before."""
+import importlib
+
+import pytest
+import torch
+
+from . import helpers as Hp
+
+F = importlib.import_module("fna2_amd.flash_naylis_attn")
+
+
+@pytest.fixture
+def native():
+    from fna2_amd import _capi
+    return _capi.native()
+
+
+def test_cpu_tensors_are_left_to_the_python_launchers(native):
+    t = torch.zeros(1, 2, 16, 64, dtype=torch.bfloat16)
+    args = (t, t, t, None, None, None, 0.1, True, None, None, 0, 0, None, False, False)
+    assert native.attn_fwd(*args) is None
+    assert native.decode(t[:, :, 0], t, t, None, None, None, 0.1, None, 0) is None
+    with pytest.raises(AssertionError, match="GPU tensor"):
+        F._fna2_forward(t, t, t, None, None, None, 0.1, True)
+
+
+CALLS = [  # dense or lengths, H, HKV, HG, D, R, causal, fp16
+    ((2, 130), 8, 4, 6, 64, 24, True, False),
+    ((1, 65), 4, 4, 0, 128, 0, False, False),
+    ((3, 200), 6, 2, 6, 128, 64, True, True),
+    ([33, 0, 257, 1], 4, 2, 3, 64, 16, True, False),
+    ([129, 40], 8, 8, 8, 128, 32, False, True),
+]
+
+
+def _both(fn, names):
+    """fn through the native path and, with it off, through the Python one."""
+    a = fn()
+    keep = {n: getattr(F, n) for n in names}
+    try:
+        for n in names:
+            setattr(F, n, lambda *x, **k: None)
+        b = fn()
+    finally:
+        for n, f in keep.items():
+            setattr(F, n, f)
+    return a, b
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("strided", [False, True])
+@pytest.mark.parametrize("call", CALLS, ids=str)
+def test_attention_bits(gpu, call, strided):
+    shape, H, HKV, HG, D, R, causal, fp16 = call
+    packed = isinstance(shape, list)
+    if packed:
+        *ins, cu, _ = Hp.make_varlen(shape, H, D, HKV, HG, R, seed=7)
+        cu = cu.to(gpu)
+        kw = dict(cu_seqlens_q=cu, cu_seqlens_k=cu, max_seqlen_q=max(shape),
+                  max_seqlen_k=max(shape))
+    else:
+        B, S = shape
+        ins = Hp.make_dense(B, H, S, D, HKV, HG, R, seed=7, layout="bshd" if strided else "bhsd")
+        kw = {}
+    ins = [t if t is None else t.to(gpu) for t in ins]
+    if fp16:
+        ins = [t if t is None or i in (3, 4, 5) else t.half() for i, t in enumerate(ins)]
+    if strided and packed:  # rows of a wider buffer
+        wide = [None if t is None or t.dim() < 2 else
+                torch.zeros(t.shape[0], t.shape[1] + 1, t.shape[2], dtype=t.dtype, device=gpu)
+                for t in ins]
+        for i, w in enumerate(wide):
+            if w is not None:
+                w[:, :ins[i].shape[1]] = ins[i]
+                ins[i] = w[:, :ins[i].shape[1]]
+    *x, dout = ins
+    leaves = [t.detach().requires_grad_(True) for t in x if t is not None]
+
+    def run():
+        it = iter(leaves)
+        a = [None if t is None else next(it) for t in x]
+        out = F.flash_naylis_attn(*a, is_causal=causal, **kw)
+        return (out, *torch.autograd.grad(out, leaves, dout))
+    assert F._native_fwd(*x, D ** -0.5, causal, **(dict(cu_q=cu, cu_k=cu) if packed else {})) \
+        is not None, "this call belongs to the native path"
+    a, b = _both(run, ["_native_fwd"])
+    c, d = _both(run, ["_native_bwd"])
+    for p, q, r, s in zip(a, b, c, d):
+        assert p.stride() == q.stride() == r.stride() == s.stride()
+        assert torch.equal(p, q) and torch.equal(p, r)
+    # without chunks (the Python launcher gives them room too): the same
+    for p, s in zip(a, d):
+        assert torch.equal(p, s)
+
+
+@pytest.mark.gpu
+def test_calls_left_to_the_python_launcher(gpu):
+    q, k, v, rq, rk, gs, dout = [t.to(gpu) for t in Hp.make_dense(1, 4, 64, 64, 4, 4, 16)]
+    s = 0.125
+    ref, _ = F._fna2_forward(q, k, v, rq, rk, gs, s, True)
+    # a feature stride of two: copied; graph_scale in bf16: converted
+    wide = torch.zeros(*q.shape[:-1], 128, dtype=q.dtype, device=gpu)
+    wide[..., ::2] = q
+    assert F._native_fwd(wide[..., ::2], k, v, rq, rk, gs, s, True) is None
+    assert torch.equal(F._fna2_forward(wide[..., ::2], k, v, rq, rk, gs, s, True)[0], ref)
+    g16 = gs.bfloat16()
+    assert F._native_fwd(q, k, v, rq, rk, g16, s, True) is None
+    F._fna2_forward(q, k, v, rq, rk, g16, s, True)
+    with pytest.raises(AssertionError, match="multiple of 8"):
+        F._fna2_forward(q, k, v, rq[..., :12].contiguous(), rk[..., :12].contiguous(), gs, s, True)
+    with pytest.raises(AssertionError, match="dtype"):
+        F._fna2_forward(q, k.half(), v, rq, rk, gs, s, True)
+    with pytest.raises(AssertionError, match="FNA2_E_SCALE"):
+        F._fna2_forward(q, k, v, rq, rk, gs, float("nan"), True)
