@@ -185,6 +185,19 @@ class DecodeArgs(ctypes.Structure):
     ]
 
 
+class DecodeRowsArgs(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int32) for n in ("batch", "heads", "heads_kv", "heads_graph",
+                                              "head_dim", "rank")] + [
+        (n, Tensor) for n in ("q", "k", "v", "r_k", "q_out", "k_out", "v_out", "rk_out")] + [
+        ("norm_q", ctypes.c_void_p),
+        ("norm_k", ctypes.c_void_p),
+        ("eps_q", ctypes.c_float),
+        ("eps_k", ctypes.c_float),
+        ("cos", ctypes.c_void_p),
+        ("sin", ctypes.c_void_p),
+    ]
+
+
 # Every symbol the header declares, with its ctypes signature.
 SIGNATURES = {
     "fna2_version": (ctypes.c_int, []),
@@ -208,6 +221,8 @@ SIGNATURES = {
     "fna2_decode_num_splits": (ctypes.c_int, [ctypes.POINTER(DecodeArgs)]),
     "fna2_decode_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(DecodeArgs)]),
     "fna2_decode": (ctypes.c_int, [ctypes.POINTER(DecodeArgs), ctypes.c_void_p]),
+    "fna2_check_decode_rows": (ctypes.c_int, [ctypes.POINTER(DecodeRowsArgs)]),
+    "fna2_decode_rows": (ctypes.c_int, [ctypes.POINTER(DecodeRowsArgs), ctypes.c_void_p]),
 }
 
 _lib = None

@@ -42,6 +42,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _capi
+from ._capi import native as _native
 from .flash_naylis_attn import BLOCK_R, flash_naylis_attn, rank_supported
 from .flash_naylis_attn import FlashNaylisAttnFunc as _FNA2Func
 from .flash_naylis_attn import _plain_eager as _fna2_plain_eager
@@ -694,11 +695,15 @@ class NaylisAttention(nn.Module):
             v = self.v_proj(x).view(B, S, self.n_kv_heads, self.head_dim).transpose(1, 2)
             if keep_rk:
                 r_q, r_k = self._rel(x)
-        if self.use_qk_norm:
-            q, k = self.q_norm(q), self.k_norm(k)
-        if self.rope is not None:
-            q, k = self.rope(q, k, position_offset=cache.length)
-        cache.append(k, v, r_k if keep_rk else None)
+        qn = self._decode_rows(q, k, v, r_k if keep_rk else None, cache) if kernel_decode else None
+        if qn is not None:
+            q = qn
+        else:
+            if self.use_qk_norm:
+                q, k = self.q_norm(q), self.k_norm(k)
+            if self.rope is not None:
+                q, k = self.rope(q, k, position_offset=cache.length)
+            cache.append(k, v, r_k if keep_rk else None)
         rows = cache.view()
         kc, vc = rows[0], rows[1]
         orig_dtype = q.dtype
@@ -715,6 +720,34 @@ class NaylisAttention(nn.Module):
             out = self._attend_eager(x, q, kc, vc, mask, rows, scale, False, False, bias)
         out = out.transpose(1, 2).contiguous().view(B, S, self.embed_dim)
         return self._finish(out, orig_dtype), (cache if use_kv_cache else None)
+
+    def _decode_rows(self, q, k, v, r_k, cache: StaticKVCache) -> Optional[torch.Tensor]:
+        """The step's QK-RMSNorm, rotation and cache append in one launch:
+        q's rows [B, H, 1, D], with the new rows in the cache; None where the
+        torch modules do it: with gradients or a tracer, in other dtypes, and
+        for a full cache or one without r_k (``append`` raises)."""
+        n = cache.length
+        if (torch.is_grad_enabled() or not _fna2_plain_eager(q) or n >= cache.capacity or
+                (cache.r_k is None) != (r_k is None)):
+            return None
+        for m, cls in ((self.q_norm, RMSNorm), (self.k_norm, RMSNorm),
+                       (self.rope, RotaryPositionalEmbedding)):
+            if m is not None and (type(m) is not cls or m._forward_hooks or m._forward_pre_hooks):
+                return None  # a replaced or hooked module is called as such
+        cos = sin = None
+        if self.rope is not None:
+            cos, sin = self.rope._table(n + 1, q.device, q.dtype)
+            cos, sin = cos[n], sin[n]
+        norm = self.use_qk_norm
+        out = _native().decode_rows(
+            q, k, v, r_k, cache.k[:, :, n:n + 1], cache.v[:, :, n:n + 1],
+            None if r_k is None else cache.r_k[:, :, n:n + 1],
+            self.q_norm.weight if norm else None, self.q_norm.eps if norm else 0.0,
+            self.k_norm.weight if norm else None, self.k_norm.eps if norm else 0.0, cos, sin)
+        if out is None:
+            return None
+        cache.length = n + 1
+        return out.unsqueeze(2)
 
     def _decode_kernel_ok(self, with_bias: bool) -> bool:
         """The decode kernel serves this head geometry (at most 32 query

@@ -1070,4 +1070,59 @@ int fna2_decode(const fna2_decode_args* a, void* stream_ptr) {
   return FNA2_OK;
 }
 
+int fna2_check_decode_rows(const fna2_decode_rows_args* a) {
+  if (!a) return FNA2_E_NULL;
+  if (a->head_dim != 64 && a->head_dim != 128) return FNA2_E_HEAD_DIM;
+  if (a->heads <= 0 || a->heads_kv <= 0 || a->heads_graph < 0) return FNA2_E_HEADS;
+  if (a->heads_graph > 0 && (a->rank < 8 || a->rank > 64 || a->rank % 8 != 0))
+    return FNA2_E_RANK;
+  if (a->batch < 0) return FNA2_E_SHAPE;
+  if ((int64_t)a->batch * ((int64_t)a->heads + 2 * (int64_t)a->heads_kv + a->heads_graph) >
+      kMaxGrid)
+    return FNA2_E_SHAPE;
+  if ((a->norm_q && !std::isfinite(a->eps_q)) || (a->norm_k && !std::isfinite(a->eps_k)))
+    return FNA2_E_SCALE;
+  if (!a->cos != !a->sin) return FNA2_E_NULL;
+  for (const void* w : {a->norm_q, a->norm_k, a->cos, a->sin})
+    if (!aligned(w, 16)) return FNA2_E_STRIDE;
+  if (a->batch == 0) return FNA2_OK;
+  for (const fna2_tensor* t : {&a->q, &a->k, &a->v, &a->q_out, &a->k_out, &a->v_out})
+    FNA2_TRY(check_bf16_rows(*t));
+  if (a->heads_graph > 0) {
+    FNA2_TRY(check_bf16_rows(a->r_k));
+    FNA2_TRY(check_bf16_rows(a->rk_out));
+  }
+  return FNA2_OK;
+}
+
+int fna2_decode_rows(const fna2_decode_rows_args* a, void* stream) {
+  FNA2_TRY(fna2_check_decode_rows(a));
+  if (a->batch == 0) return FNA2_OK;
+  FNA2_TRY(check_device());
+  fna2::DecodeRowsParams K;
+  std::memset(&K, 0, sizeof(K));
+  K.B = a->batch;
+  K.H = a->heads;
+  K.H_KV = a->heads_kv;
+  K.H_G = a->heads_graph;
+  K.D = a->head_dim;
+  K.R = a->heads_graph > 0 ? a->rank : 0;
+  K.q = view(a->q);
+  K.k = view(a->k);
+  K.v = view(a->v);
+  K.rk = view(a->r_k);
+  K.qo = view(a->q_out);
+  K.ko = view(a->k_out);
+  K.vo = view(a->v_out);
+  K.rko = view(a->rk_out);
+  K.wq = (const uint16_t*)a->norm_q;
+  K.wk = (const uint16_t*)a->norm_k;
+  K.eps_q = a->eps_q;
+  K.eps_k = a->eps_k;
+  K.cos = (const uint16_t*)a->cos;
+  K.sin = (const uint16_t*)a->sin;
+  if (fna2::launch_decode_rows(K, (hipStream_t)stream) != hipSuccess) return FNA2_E_LAUNCH;
+  return FNA2_OK;
+}
+
 }  // extern "C"

@@ -122,6 +122,17 @@ struct DecodeParams {
   float* acc;  // nsplit > 1: [nsplit][B][H][D] unnormalised numerators
   float* ml;   // nsplit > 1: [nsplit][B][H] (max, sum) pairs
 };
+// The new token's rows of a decode step (fna2_decode.hip).
+struct DecodeRowsParams {
+  int B, H, H_KV, H_G, D, R;
+  TView q, k, v, rk, qo, ko, vo, rko;
+  const uint16_t* wq;  // bf16 [D], or null
+  const uint16_t* wk;
+  float eps_q, eps_k;
+  const uint16_t* cos;  // bf16 [D], or null
+  const uint16_t* sin;
+};
+hipError_t launch_decode_rows(const DecodeRowsParams& P, hipStream_t s);
 constexpr int kDecodeStages = 2;  // LDS ring depth of a decode wave
 // Rank-tile chunks of a decode kernel for `rch` used chunks (graph heads of
 // a group x R / 8): 0, 4, 8, 16 or 32; -1 if too wide.

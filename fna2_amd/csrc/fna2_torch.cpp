@@ -42,6 +42,7 @@ struct Lib {
   decltype(&fna2_decode) decode;
   decltype(&fna2_decode_workspace_bytes) decode_workspace_bytes;
   decltype(&fna2_check_decode) check_decode;
+  decltype(&fna2_decode_rows) decode_rows;
   decltype(&fna2_rope_varlen) rope_varlen;
   decltype(&fna2_rope_bwd) rope_bwd;
   decltype(&fna2_rope_bwd_workspace_bytes) rope_bwd_workspace_bytes;
@@ -58,6 +59,7 @@ void bind(const std::map<std::string, uintptr_t>& f) {
   FNA2_BIND(decode);
   FNA2_BIND(decode_workspace_bytes);
   FNA2_BIND(check_decode);
+  FNA2_BIND(decode_rows);
   FNA2_BIND(rope_varlen);
   FNA2_BIND(rope_bwd);
   FNA2_BIND(rope_bwd_workspace_bytes);
@@ -295,7 +297,8 @@ std::optional<std::tuple<Tensor, Tensor>> decode(const Tensor& q_, const Tensor&
                                                  const OptTensor& rkc_, const OptTensor& gs_,
                                                  double scale, const OptTensor& seq_,
                                                  int64_t num_splits) {
-  const Tensor &rkc = opt(rkc_), &gs = opt(gs_), &seq = opt(seq_);
+  const Tensor &rkc = opt(rkc_), &seq = opt(seq_);
+  Tensor gs = opt(gs_);
   if (!L.decode || !q_.defined() || !q_.is_cuda()) return std::nullopt;
   const c10::Device dev = q_.device();
   // [B, H, F], or [B, H, 1, F] with the row dimension dropped
@@ -334,7 +337,10 @@ std::optional<std::tuple<Tensor, Tensor>> decode(const Tensor& q_, const Tensor&
     return v;
   };
   if (rq_.has_value()) {
-    if (!row(*rq_, rq) || rq.size(0) != B || !rkc.defined() || !gs.defined()) return std::nullopt;
+    if (!row(*rq_, rq) || rq.size(0) != B || !rkc.defined() || !plain(gs, dev) ||
+        !gs.is_floating_point())
+      return std::nullopt;
+    gs = gs.detach().to(at::kFloat).contiguous();  // (a module's parameter is bf16)
     if (!cache(rkc, B, rq.size(2)) || rkc.size(1) != rq.size(1) || rkc.size(2) != kc.size(2) ||
         !float_on(gs, dev, rq.size(1)))
       return std::nullopt;
@@ -366,6 +372,74 @@ std::optional<std::tuple<Tensor, Tensor>> decode(const Tensor& q_, const Tensor&
   }
   if (L.decode(&a, stream_of(dev)) != FNA2_OK) return std::nullopt;
   return std::make_tuple(out, lse);
+}
+
+// The rows of a decode step: normalised and rotated q as [B, H, D]; k, v and
+// r_k into k_out, v_out and rk_out.  All [B, heads, 1, F]; norm weights and
+// the cos / sin rows [D], bf16.  None, with nothing written: not this call.
+OptTensor decode_rows(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& rk_,
+                      const Tensor& k_out, const Tensor& v_out, const OptTensor& rko_,
+                      const OptTensor& nq, double eps_q, const OptTensor& nk, double eps_k,
+                      const OptTensor& cos, const OptTensor& sin) {
+  if (!L.decode_rows || !q.defined() || !q.is_cuda()) return std::nullopt;
+  const c10::Device dev = q.device();
+  auto rows = [&](const Tensor& t) {
+    return plain(t, dev) && t.scalar_type() == at::kBFloat16 && t.dim() == 4 && t.size(2) == 1 &&
+           t.size(0) == q.size(0) && rows16(t);
+  };
+  if (!rows(q)) return std::nullopt;
+  const int64_t D = q.size(3);
+  for (const Tensor* t : {&k, &v, &k_out, &v_out})
+    if (!rows(*t) || t->sizes() != k.sizes()) return std::nullopt;
+  if (k.size(3) != D || rk_.has_value() != rko_.has_value()) return std::nullopt;
+  fna2_decode_rows_args a{};
+  auto vec = [&](const OptTensor& t, const void*& p) {
+    if (!t.has_value()) return true;
+    if (!plain(*t, dev) || t->scalar_type() != at::kBFloat16 || !t->is_contiguous() ||
+        t->numel() != D || (uintptr_t)t->data_ptr() % 16)
+      return false;
+    p = t->data_ptr();
+    return true;
+  };
+  if (!vec(nq, a.norm_q) || !vec(nk, a.norm_k) || !vec(cos, a.cos) || !vec(sin, a.sin))
+    return std::nullopt;
+  auto row_view = [](const Tensor& t) {
+    fna2_tensor v{};
+    v.ptr = t.data_ptr();
+    v.stride_b = t.stride(0);
+    v.stride_h = t.stride(1);
+    return v;
+  };
+  a.batch = (int32_t)q.size(0);
+  a.heads = (int32_t)q.size(1);
+  a.heads_kv = (int32_t)k.size(1);
+  a.head_dim = (int32_t)D;
+  if (rk_.has_value()) {
+    if (!rows(*rk_) || !rows(*rko_) || rk_->sizes() != rko_->sizes()) return std::nullopt;
+    a.heads_graph = (int32_t)rk_->size(1);
+    a.rank = (int32_t)rk_->size(3);
+    a.r_k = row_view(*rk_);
+    a.rk_out = row_view(*rko_);
+  }
+  // The cache rows are written in place, as torch's copy_ would: an inference
+  // tensor only in inference mode, any other with its version counted up.
+  const Tensor* written[3] = {&k_out, &v_out, rko_.has_value() ? &*rko_ : nullptr};
+  for (const Tensor* t : written)
+    if (t && t->is_inference() && !c10::InferenceMode::is_enabled()) return std::nullopt;
+  const c10::DeviceGuard guard(dev);
+  const Tensor out = at::empty({q.size(0), q.size(1), D}, q.options());
+  a.q = row_view(q);
+  a.k = row_view(k);
+  a.v = row_view(v);
+  a.q_out = row_view(out);
+  a.k_out = row_view(k_out);
+  a.v_out = row_view(v_out);
+  a.eps_q = (float)eps_q;
+  a.eps_k = (float)eps_k;
+  if (L.decode_rows(&a, stream_of(dev)) != FNA2_OK) return std::nullopt;
+  for (const Tensor* t : written)
+    if (t && !t->is_inference()) t->unsafeGetTensorImpl()->bump_version();
+  return out;
 }
 
 // The arguments rope_varlen's forward and backward share.  w: the norm
@@ -471,6 +545,7 @@ PYBIND11_MODULE(_torch_binding, m) {
   m.def("attn_fwd", &attn_fwd, Free());
   m.def("attn_bwd", &attn_bwd, Free());
   m.def("decode", &decode, Free());
+  m.def("decode_rows", &decode_rows, Free());
   m.def("rope_fwd", &rope_fwd, Free());
   m.def("rope_bwd", &rope_bwd, Free());
 }

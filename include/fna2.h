@@ -288,6 +288,29 @@ size_t fna2_decode_workspace_bytes(const fna2_decode_args* args);
  * split.  Writes out (and lse). */
 int fna2_decode(const fna2_decode_args* args, void* hip_stream);
 
+/* The rows of a decode step, in one launch: one new token per sequence, q
+ * [B, H, D], k and v [B, H_KV, D] and r_k [B, H_G, R] as a projection wrote
+ * them (row views as in fna2_decode_args).  q and k rows are RMS-normalised
+ * (optional: x rsqrt(mean(x^2) + eps) w) and rotated by the given cos / sin
+ * rows (optional: y_i = x_i cos_i - x_{i+D/2} sin_i, y_{i+D/2} =
+ * x_{i+D/2} cos_{i+D/2} + x_i sin_{i+D/2}), in fp32 with one rounding after
+ * each; k, v and r_k go to their cache rows.  bf16. */
+typedef struct fna2_decode_rows_args {
+  int32_t batch, heads, heads_kv, heads_graph, head_dim, rank;
+  fna2_tensor q, k, v, r_k;                 /* inputs (r_k: heads_graph > 0) */
+  fna2_tensor q_out, k_out, v_out, rk_out;  /* written; disjoint from every input */
+  const void* norm_q;  /* [D] bf16, or NULL: q not normalised */
+  const void* norm_k;
+  float eps_q, eps_k;
+  const void* cos;     /* [D] bf16, both or neither NULL (no rotation) */
+  const void* sin;
+} fna2_decode_rows_args;
+
+/* Host-only validation; no GPU call. */
+int fna2_check_decode_rows(const fna2_decode_rows_args* args);
+
+int fna2_decode_rows(const fna2_decode_rows_args* args, void* hip_stream);
+
 /* ABI version (FNA2_ABI_VERSION). */
 int fna2_version(void);
 
