@@ -918,6 +918,7 @@ namespace {
 // (a fixed figure, so that the split count and the workspace size are a
 // function of the arguments alone).
 constexpr int kDecodeCUs = 256;
+constexpr int64_t kDecodeFewWaves = 2 * kDecodeCUs;
 constexpr int64_t kOff31 = ((int64_t)1 << 31) - 16;  // buffer-offset bound
 
 int dec_group(const fna2_decode_args& a) { return a.heads / a.heads_kv; }
@@ -954,7 +955,17 @@ DecSplit dec_split(const fna2_decode_args& a) {
                                                    fna2::decode_stage_bytes(a.head_dim, rc)));
     const int64_t target = 2ll * kDecodeCUs * per_cu;  // two rounds of resident waves
     n = std::min<int64_t>(cdiv64(target, units), cdiv64(L, 128));  // >= 4 steps a split
+    // Few units: a split's steps are a chain of load latencies that nothing
+    // else hides, so down to one step each as long as the waves stay few (two
+    // per CU; more and the merge and the waves' own start outweigh it).  Up
+    // to two steps a second launch costs more than it saves.  Measured (decode
+    // and merge, us, four-step splits -> the rule's): B2 H8/4 L496 d128 13.0 ->
+    // 9.0, B1 H16 L200 d64 10.0 -> 7.7, B1 H32/8 L4096 d128 10.7 -> 9.7; B1 H8
+    // L64 6.4 whole, 8.3 in two; B4 H32/8 L2500: 20 splits (640 waves) 12.2,
+    // 40 15.8.
+    if (L > 64) n = std::max<int64_t>(n, std::min<int64_t>(kDecodeFewWaves / units, cdiv64(L, 32)));
     n = std::max<int64_t>(std::min<int64_t>(n, 64), 1);
+    if (L <= 64) n = 1;
   }
   n = std::min<int64_t>(n, cdiv64(L, 32));
   s.keys = (int)(cdiv64(cdiv64(L, n), 32) * 32);

@@ -37,6 +37,8 @@
 // (max, sum) pair to the workspace, and the merge kernel combines them into
 //     O = sum_s e^{c (m_s - M)} acc_s / (sum_s e^{c (m_s - M)} l_s + 1e-6),
 // the forward kernel's normalisation (FNA2/flash_naylis_attn.py:192-195).
+#include <algorithm>
+
 #include "fna2_kernels.h"
 #include "fna2_tile.h"
 
@@ -300,53 +302,79 @@ __device__ __forceinline__ void decode_body(const DecodeParams& P) {
   if (hl == 0) *(f32x2*)(P.ml + 2 * row) = f32x2{m_i, l_tot};
 }
 
-// One wave per (sequence, head): combine the splits' partial results.
+// One workgroup per (sequence, head) combines the splits' partial results.
+// A row of D fp32 values is 16 bytes for each of D / 4 lanes, so a wave reads
+// 256 / D splits at once and the four waves 4 of those, kMergeAhead deep:
+// the loads of 40 splits are all in flight together.  (One wave per row,
+// one split after the other, was a chain of nsplit loads: 7.0 us for 20
+// splits of 128 rows; decode and merge of 4 sequences of 2500 rows, H32/8
+// d128: 17.3 -> 12.5 us.)  The sum's order depends on nsplit alone.
+constexpr int kMergeAhead = 4;
 template <int D>
 __device__ __forceinline__ void merge_body(const DecodeParams& P) {
-  const int lane = threadIdx.x & 63;
-  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);  // b * H + h
-  if (r >= (int64_t)P.B * P.H) return;
-  const int b = (int)(r / P.H), h = (int)(r % P.H);
+  constexpr int LPR = D / 4, SPW = 64 / LPR, SPB = 4 * SPW;  // lanes a row; splits a wave, a block
+  __shared__ float part[4][D];
+  const int lane = threadIdx.x & 63, wv = uni(threadIdx.x >> 6);
   const int64_t plane = (int64_t)P.B * P.H;  // rows per split
-  float m = kNegInf, l = 0.f;
-  if (lane < P.nsplit) {
-    const f32x2 ml = *(const f32x2*)(P.ml + 2 * (lane * plane + r));
-    m = ml[0];
-    l = ml[1];
-  }
-  float M = m;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off));
-  const float w = (m == kNegInf) ? 0.f : __builtin_amdgcn_exp2f((m - M) * P.c2);
-  float L = l * w;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off);
-  constexpr int E = D / 64;  // features per lane
-  float o[E];
-#pragma unroll
-  for (int e = 0; e < E; ++e) o[e] = 0.f;
-  for (int s = 0; s < P.nsplit; ++s) {
-    const float ws = __shfl(w, s);
-    const float* a = P.acc + (s * plane + r) * D + lane * E;
-    if constexpr (E == 2) {
-      const f32x2 x = *(const f32x2*)a;
-      o[0] += ws * x[0];
-      o[1] += ws * x[1];
-    } else {
-#pragma unroll
-      for (int e = 0; e < E; ++e) o[e] += ws * a[e];
+  for (int64_t r = blockIdx.x; r < plane; r += gridDim.x) {  // b * H + h
+    const int b = (int)(r / P.H), h = (int)(r % P.H);
+    const int s0 = wv * SPW + lane / LPR, f = 4 * (lane % LPR);
+    const float* src = P.acc + r * D + f;
+    f32x4_t x[kMergeAhead];
+  #pragma unroll
+    for (int j = 0; j < kMergeAhead; ++j) {
+      const int s = s0 + j * SPB;
+      x[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (s < P.nsplit) x[j] = *(const f32x4_t*)(src + s * plane * D);
     }
-  }
-  const float inv = 1.f / (L + 1e-6f);
-  uint16_t* orow = (uint16_t*)P.o.ptr + (int64_t)b * P.o.sb + (int64_t)h * P.o.sh + lane * E;
-  if constexpr (E == 2) {
-    *(uint32_t*)orow = pack_bf16(o[0] * inv, o[1] * inv);
-  } else {
-    orow[0] = (uint16_t)(pack_bf16(o[0] * inv, 0.f) & 0xffffu);
-  }
-  if (lane == 0 && P.lse.ptr) {
-    float* lrow = (float*)P.lse.ptr + (int64_t)b * P.lse.sb + (int64_t)h * P.lse.sh;
-    *lrow = (M == kNegInf) ? kNegInf : M * P.c + __builtin_amdgcn_logf(L + 1e-6f) * kLn2;
+    float m = kNegInf, l = 0.f;
+    if (lane < P.nsplit) {
+      const f32x2 ml = *(const f32x2*)(P.ml + 2 * (lane * plane + r));
+      m = ml[0];
+      l = ml[1];
+    }
+    float M = m;
+  #pragma unroll
+    for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off));
+    const float w = (m == kNegInf) ? 0.f : __builtin_amdgcn_exp2f((m - M) * P.c2);
+    float L = l * w;
+  #pragma unroll
+    for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off);
+    f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+    for (int base = 0; base < P.nsplit; base += kMergeAhead * SPB) {
+  #pragma unroll
+      for (int j = 0; j < kMergeAhead; ++j) {
+        const int s = base + s0 + j * SPB;
+        const float ws = __shfl(w, s & 63);
+        if (s < P.nsplit) o += ws * x[j];
+      }
+  #pragma unroll
+      for (int j = 0; j < kMergeAhead; ++j) {  // the next round, if any
+        const int s = base + s0 + (kMergeAhead + j) * SPB;
+        if (s < P.nsplit) x[j] = *(const f32x4_t*)(src + s * plane * D);
+      }
+    }
+  #pragma unroll
+    for (int off = LPR; off < 64; off <<= 1)
+  #pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] += __shfl_xor(o[i], off);
+    if (lane < LPR) *(f32x4_t*)(&part[wv][f]) = o;
+    __syncthreads();
+    const float inv = 1.f / (L + 1e-6f);
+    if (threadIdx.x < D / 2) {
+      const int d = 2 * threadIdx.x;
+      float y[2];
+  #pragma unroll
+      for (int i = 0; i < 2; ++i)
+        y[i] = (part[0][d + i] + part[1][d + i] + part[2][d + i] + part[3][d + i]) * inv;
+      uint16_t* orow = (uint16_t*)P.o.ptr + (int64_t)b * P.o.sb + (int64_t)h * P.o.sh;
+      *(uint32_t*)(orow + d) = pack_bf16(y[0], y[1]);
+    }
+    if (threadIdx.x == 0 && P.lse.ptr) {
+      float* lrow = (float*)P.lse.ptr + (int64_t)b * P.lse.sb + (int64_t)h * P.lse.sh;
+      *lrow = (M == kNegInf) ? kNegInf : M * P.c + __builtin_amdgcn_logf(L + 1e-6f) * kLn2;
+    }
+    __syncthreads();  // `part` is read: the next row may write it
   }
 }
 
@@ -488,7 +516,7 @@ hipError_t launch_decode_merge(const DecodeParams& P, hipStream_t s) {
   if (rows <= 0 || P.nsplit <= 1) return hipSuccess;
   void (*k)(const DecodeParams) = P.D == 64 ? decode_merge_d64 : P.D == 128 ? decode_merge_d128 : nullptr;
   if (!k) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k, dim3((uint32_t)((rows + 3) / 4)), dim3(256), 0, s, P);
+  hipLaunchKernelGGL(k, dim3((uint32_t)std::min<int64_t>(rows, 1 << 16)), dim3(256), 0, s, P);
   return hipGetLastError();
 }
 

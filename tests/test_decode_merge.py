@@ -1,0 +1,58 @@
+"""The decode's split rule for few units, and the merge of the splits at the
+counts where its rounds and waves change (fna2_decode.hip merge_body)."""
+import ctypes
+
+import pytest
+import torch
+
+from fna2_amd import _capi
+
+
+def _splits(B, H, HKV, HG, D, R, L):
+    a = _capi.DecodeArgs()
+    a.batch, a.heads, a.heads_kv, a.heads_graph = B, H, HKV, HG
+    a.head_dim, a.rank, a.max_seqlen_k, a.softmax_scale = D, R, L, 0.1
+    fake = 1 << 20
+    for n in ("q", "r_q", "k_cache", "v_cache", "rk_cache", "out"):
+        setattr(a, n, _capi.Tensor(fake, 1 << 20, 128, 1 << 14))
+    a.graph_scale = fake
+    return _capi.lib().fna2_decode_num_splits(ctypes.byref(a))
+
+
+@pytest.mark.parametrize("L,n", [(0, 1), (1, 1), (64, 1), (65, 3), (96, 3), (97, 4), (2048, 64),
+                                 (4096, 64)])
+def test_few_units_split_to_single_steps(L, n):
+    assert _splits(1, 8, 8, 0, 128, 0, L) == n
+
+
+def test_many_units_keep_long_splits():
+    assert _splits(64, 16, 16, 16, 128, 32, 4096) <= 3
+    assert _splits(64, 16, 16, 16, 128, 32, 128) == 1
+    assert _splits(8, 32, 8, 0, 128, 0, 1024) == 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,R", [(64, 16), (128, 32)])
+@pytest.mark.parametrize("n", [2, 7, 8, 9, 16, 17, 31, 32, 33, 63, 64])
+def test_merge_of_n_splits(gpu, n, D, R):
+    from fna2_amd.decode import flash_naylis_decode
+    print(n, D, R, flush=True)
+    B, H, HKV, HG, L = 3, 6, 2, 4, 64 * 32
+    g = torch.Generator().manual_seed(n + D)
+    mk = lambda *s, f=1.0: (torch.randn(*s, generator=g) * f).bfloat16().to(gpu)
+    q, k, v = mk(B, H, D), mk(B, HKV, L, D), mk(B, HKV, L, D)
+    rq, rk = mk(B, HG, R, f=R ** -0.5), mk(B, HG, L, R, f=R ** -0.5)
+    gs = torch.ones(HG, device=gpu)
+    seq = torch.tensor([L, 33, 0], dtype=torch.int32, device=gpu)  # splits with no rows
+    run = lambda s: flash_naylis_decode(q, k, v, rq, rk, gs, cache_seqlens=seq, num_splits=s,
+                                        return_lse=True)
+    (o, l), (o1, l1) = run(n), run(1)
+    torch.cuda.synchronize()
+    # P is rounded to bf16 against each split's own maximum: 2^-9 of each of
+    # the terms, so of the output's scale; the LSE is an fp32 sum
+    assert (o.float() - o1.float()).abs().max() <= 2 ** -7 * o1.float().abs().max()
+    fin = torch.isfinite(l1)
+    assert torch.equal(torch.isfinite(l), fin) and not fin[2].any()
+    assert (l - l1)[fin].abs().max() < 1e-5
+    assert not o[2].any()
+    assert torch.equal(run(n)[0], o)
