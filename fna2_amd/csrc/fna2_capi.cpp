@@ -823,7 +823,7 @@ void rope_out(fna2::RopeParams& P, const fna2_tensor& qo, const fna2_tensor& ko)
 
 size_t rope_ws(const fna2_rope_args* a) {
   if (!(a->norm_q || a->norm_k) || rope_empty(a)) return 0;
-  return align_up(sizeof(float) * 2u * (size_t)fna2::rope_blocks(a->total_tokens) *
+  return align_up(sizeof(float) * 2u * (size_t)fna2::rope_bwd_blocks(a->total_tokens) *
                   (size_t)a->head_dim);
 }
 

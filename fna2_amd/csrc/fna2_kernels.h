@@ -84,6 +84,7 @@ inline int padded_rank32(int H_G, int R) {
 constexpr int kRopeBF16 = 1, kRopeF16 = 2, kRopeF32 = 3;
 struct RopeParams {
   int dtype, T, Hq, Hk, D, nseq, sign;
+  int tpw;  // consecutive tokens per wave (set by the launches)
   const int* cu;         // [nseq + 1]
   const float* inv_freq;  // [D / 2]
   const void* q;
@@ -95,7 +96,7 @@ struct RopeParams {
   const float* wk;
   float eps;
   // backward of the normalised rotation: incoming gradients, dw partials
-  // [2][rope_blocks(T)][D] and the weight gradients
+  // [2][rope_bwd_blocks(T)][D] and the weight gradients
   const void* gq;
   const void* gk;
   int64_t gq_ss, gq_sh, gk_ss, gk_sh;
@@ -103,7 +104,7 @@ struct RopeParams {
   float* dwq;
   float* dwk;
 };
-int rope_blocks(int T);  // workgroups of a rotary launch over T tokens
+int rope_bwd_blocks(int T);  // workgroups of the norm backward over T tokens
 hipError_t launch_rope(const RopeParams& P, hipStream_t s);
 hipError_t launch_rope_norm_bwd(const RopeParams& P, hipStream_t s);
 

@@ -22,8 +22,8 @@
 // owns 16 bytes of the row's first half and the matching 16 bytes of its
 // second half; the lanes of a wave cover 64 / LPR rows at a time, and the
 // lane keeps the cos/sin of its 16-byte column range for all the token's
-// heads (computed once per token).  A workgroup covers 16 consecutive
-// tokens (4 per wave); the sequence of a wave's first token comes from a
+// heads (computed once per token).  A workgroup covers 4 to 16 consecutive
+// tokens; the sequence of a wave's first token comes from a
 // binary search of cu_seqlens, later ones by stepping.
 #include "fna2_kernels.h"
 
@@ -31,10 +31,18 @@ namespace fna2 {
 
 namespace {
 
-constexpr int kRopeTokensPerWave = 4;
 constexpr int kRopeWaves = 4;
 constexpr int kRopePasses = 4;  // row passes whose loads are in flight together
-constexpr int kBwdPasses = 2;   // (the norm backward holds twice the data per pass)
+// The norm backward reads two tensors and is bound by how many loads the CU
+// has in flight: its rows stay raw words until used and the norm weights
+// stay in LDS, so that four waves share a SIMD (two with fp32 rows and the
+// weights in registers).  Passes in flight per wave, 16-bit and fp32: with
+// 16-bit rows a second one no longer fits four waves' registers (c3 pack: 90.6
+// us; two passes at three waves 98, four at two 109; before, 104.  fp32, 6000
+// tokens: two passes 66, one 73; before, 84).
+constexpr int kBwdOcc = 4;
+template <int DT>
+constexpr int kBwdPasses = DT == kRopeF32 ? 2 : 1;
 
 // Products and sums that are never fused into a multiply-add (the
 // reference evaluates them as separate elementwise ops).
@@ -127,7 +135,7 @@ struct Raw {
 
 // Lane layout and the token -> sequence walk shared by the kernels: lane
 // owns columns [col, col + EPL) of both halves of row lrow + j * rpw of a
-// token; a wave covers kRopeTokensPerWave consecutive tokens from t0.
+// token; a wave covers P.tpw consecutive tokens from t0.
 template <int DT>
 struct RopeLanes {
   static constexpr int EPL = Chunk<DT>::EPL;
@@ -140,7 +148,7 @@ struct RopeLanes {
     col = (lane % lpr) * EPL;
     lrow = lane / lpr;
     nrows = P.Hq + P.Hk;
-    t0 = wave_id * kRopeTokensPerWave;
+    t0 = wave_id * P.tpw;
     // Largest b with cu[b] <= t0 (b = -1: before the first sequence).
     const auto cu = const_space(P.cu);
     const int n = P.nseq;
@@ -174,6 +182,47 @@ struct RopeLanes {
   }
 };
 
+// cos and sin of a token's D / 2 angles, each formed by one lane of the wave
+// and handed to the others through LDS: the 64 / lpr rows of a wave pass
+// share their columns, so forming them where they are used repeats every
+// sincosf 64 / lpr times (8 at d = 128 in bf16).  TD: the type the table is
+// rounded to.  (c3 pack, 16384 tokens x 32 heads of 128, bf16: norm backward
+// 108 -> 104 us; the forward, bound by its stores, unchanged at 50.)
+constexpr int kMaxHalf = 256;
+template <int TD, int EPL>
+struct RopeTable {
+  float* cos;  // this wave's [kMaxHalf], then sin
+  float invf[kMaxHalf / 64];
+  __device__ __forceinline__ RopeTable(const RopeParams& P, float* lds, int lane, int half)
+      : cos(lds) {
+#pragma unroll
+    for (int k = 0; k < kMaxHalf / 64; ++k)
+      invf[k] = lane + 64 * k < half ? rnd<TD>(P.inv_freq[lane + 64 * k]) : 0.f;
+  }
+  // Position p's cos and sin (times `sign`) of columns col .. col + EPL - 1.
+  __device__ __forceinline__ void at(int p, int sign, int lane, int half, int col,
+                                     float (&c)[EPL], float (&s)[EPL]) const {
+    const float pos = rnd<TD>((float)p);
+    float* sin = cos + kMaxHalf;
+#pragma unroll
+    for (int k = 0; k < kMaxHalf / 64; ++k) {
+      if (lane + 64 * k < half) {
+        float sv, cv;
+        sincosf(rnd<TD>(mul_rn(pos, invf[k])), &sv, &cv);  // the accurate library routine
+        cos[lane + 64 * k] = rnd<TD>(cv);
+        sin[lane + 64 * k] = sign * rnd<TD>(sv);
+      }
+    }
+    // (one wave's own LDS: its reads follow its writes in order)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) c[e] = cos[col + e], s[e] = sin[col + e];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+};
+
 // Sum over the lpr lanes of a row (lanes lrow * lpr .. + lpr - 1); every
 // lane of the wave takes part.
 __device__ __forceinline__ float row_sum(float v, int lpr) {
@@ -190,14 +239,14 @@ __global__ __launch_bounds__(64 * kRopeWaves) void rope_kernel(const RopeParams 
   constexpr int EPL = Ch::EPL;
   constexpr int ES = DT == kRopeF32 ? 4 : 2;
   constexpr int TD = NORM ? kRopeF32 : DT;  // type of the table and of the rotation
-  RopeLanes<DT> L(P, blockIdx.x * kRopeWaves + uni(threadIdx.x >> 6));
+  const int wv = uni(threadIdx.x >> 6);
+  RopeLanes<DT> L(P, blockIdx.x * kRopeWaves + wv);
   // (no early return before the weights' barrier: a wave past the last
   // token runs no token iteration below)
   const int col = L.col, half = L.half;
 
-  float invf[EPL];
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) invf[e] = rnd<TD>(P.inv_freq[col + e]);
+  __shared__ __attribute__((aligned(16))) float table[kRopeWaves][2 * kMaxHalf];
+  const RopeTable<TD, EPL> tab(P, table[wv], L.lane, half);
   // the norm weights (q, k), in LDS rather than in every lane's registers
   __shared__ float wsh[NORM ? 2 : 1][NORM ? 512 : 1];
   if constexpr (NORM) {
@@ -209,23 +258,13 @@ __global__ __launch_bounds__(64 * kRopeWaves) void rope_kernel(const RopeParams 
   }
   const float inv_d = 1.f / (float)P.D;
 
-  for (int i = 0; i < kRopeTokensPerWave; ++i) {
+  for (int i = 0; i < P.tpw; ++i) {
     const int t = L.t0 + i;
     if (t >= P.T) break;
     const int p = L.position(P, t);
     const bool inside = p >= 0;
     float c[EPL], s[EPL];
-    if (inside) {
-      const float pos = rnd<TD>((float)p);
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        const float ang = rnd<TD>(mul_rn(pos, invf[e]));
-        float sv, cv;
-        sincosf(ang, &sv, &cv);  // the accurate library routine
-        c[e] = rnd<TD>(cv);
-        s[e] = P.sign * rnd<TD>(sv);
-      }
-    }
+    if (inside) tab.at(p, P.sign, L.lane, half, col, c, s);
     // Four row passes at a time: every load first, then the arithmetic and
     // the stores.  (With the norm every lane makes the same passes: the row
     // sums cross lanes.)
@@ -302,104 +341,106 @@ __global__ __launch_bounds__(64 * kRopeWaves) void rope_kernel(const RopeParams 
 // outside every sequence pass dy through.  Each workgroup writes its dw
 // partial sums (fixed order) to part[2][gridDim.x][D].
 template <int DT>
-__global__ __launch_bounds__(64 * kRopeWaves) void rope_norm_bwd_kernel(const RopeParams P) {
+__global__ __launch_bounds__(64 * kRopeWaves, kBwdOcc) void rope_norm_bwd_kernel(const RopeParams P) {
   using Ch = Chunk<DT>;
   constexpr int EPL = Ch::EPL;
   constexpr int ES = DT == kRopeF32 ? 4 : 2;
-  __shared__ float red[2][kRopeWaves][512];
+  constexpr int NP = kBwdPasses<DT>;
+  __shared__ __attribute__((aligned(16))) float red[2][kRopeWaves][512];
+  __shared__ __attribute__((aligned(16))) float table[kRopeWaves][2 * kMaxHalf];
+  __shared__ __attribute__((aligned(16))) float wsh[2][512];
   const int wv = uni(threadIdx.x >> 6);
   RopeLanes<DT> L(P, blockIdx.x * kRopeWaves + wv);
   const int col = L.col, half = L.half, lane = L.lane;
-  float invf[EPL], wq1[EPL], wq2[EPL], wk1[EPL], wk2[EPL];
-  float aq1[EPL], aq2[EPL], ak1[EPL], ak2[EPL];  // dw partials of this lane's columns
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) {
-    invf[e] = P.inv_freq[col + e];
-    wq1[e] = P.wq ? P.wq[col + e] : 1.f;
-    wq2[e] = P.wq ? P.wq[half + col + e] : 1.f;
-    wk1[e] = P.wk ? P.wk[col + e] : 1.f;
-    wk2[e] = P.wk ? P.wk[half + col + e] : 1.f;
-    aq1[e] = aq2[e] = ak1[e] = ak2[e] = 0.f;
+  const RopeTable<kRopeF32, EPL> tab(P, table[wv], lane, half);
+  for (int d = threadIdx.x; d < P.D; d += 64 * kRopeWaves) {
+    wsh[0][d] = P.wq ? P.wq[d] : 1.f;
+    wsh[1][d] = P.wk ? P.wk[d] : 1.f;
   }
+  __syncthreads();
+  float dw1[2][EPL], dw2[2][EPL];  // dw partials of this lane's columns (q, k)
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) dw1[0][e] = dw2[0][e] = dw1[1][e] = dw2[1][e] = 0.f;
   const float inv_d = 1.f / (float)P.D;
 
-  for (int i = 0; i < kRopeTokensPerWave && L.t0 < P.T; ++i) {
+  for (int i = 0; i < P.tpw && L.t0 < P.T; ++i) {
     const int t = L.t0 + i;
     if (t >= P.T) break;
     const int p = L.position(P, t);
     const bool inside = p >= 0;
     float c[EPL], s[EPL];
-    if (inside) {
-      const float pos = (float)p;
+    if (inside) tab.at(p, P.sign, lane, half, col, c, s);
+    // The q rows, then the k rows: one side's weights and pointers at a time.
+    static_for<2>([&](auto side_) {
+      constexpr int side = decltype(side_)::value;
+      const int rows = side ? P.Hk : P.Hq;
+      const bool has_w = (side ? P.wk : P.wq) != nullptr;
+      const char* xs = (const char*)(side ? P.k : P.q) + (int64_t)t * (side ? P.k_ss : P.q_ss) * ES;
+      const char* gs = (const char*)(side ? P.gk : P.gq) + (int64_t)t * (side ? P.gk_ss : P.gq_ss) * ES;
+      char* os = (char*)(side ? P.k_out : P.q_out) + (int64_t)t * (side ? P.ko_ss : P.qo_ss) * ES;
+      const int64_t xh = (side ? P.k_sh : P.q_sh) * ES, gh = (side ? P.gk_sh : P.gq_sh) * ES;
+      const int64_t oh = (side ? P.ko_sh : P.qo_sh) * ES;
+      for (int r0 = L.lrow; r0 - L.lrow < rows; r0 += NP * L.rpw) {
+        // every load of NP row passes first, as raw words
+        Raw<DT> x1[NP], x2[NP], g1[NP], g2[NP];
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        float sv, cv;
-        sincosf(mul_rn(pos, invf[e]), &sv, &cv);
-        c[e] = cv;
-        s[e] = P.sign * sv;
-      }
-    }
-    for (int r0 = L.lrow; r0 - L.lrow < L.nrows; r0 += kBwdPasses * L.rpw) {
-      Ch x1[kBwdPasses], x2[kBwdPasses], g1[kBwdPasses], g2[kBwdPasses];
-      char* dst[kBwdPasses];
-      bool isq[kBwdPasses];
-#pragma unroll
-      for (int j = 0; j < kBwdPasses; ++j) {
-        const int r = r0 + j * L.rpw;
-        dst[j] = nullptr;
-        isq[j] = r < P.Hq;
-        if (r < L.nrows) {
-          const char* xs = L.in_row(P, P.q, P.k, P.q_ss, P.q_sh, P.k_ss, P.k_sh, t, r);
-          const char* gs = L.in_row(P, P.gq, P.gk, P.gq_ss, P.gq_sh, P.gk_ss, P.gk_sh, t, r);
-          dst[j] = (char*)L.in_row(P, P.q_out, P.k_out, P.qo_ss, P.qo_sh, P.ko_ss, P.ko_sh, t, r);
-          x1[j].load(xs + col * ES);
-          x2[j].load(xs + (half + col) * ES);
-          g1[j].load(gs + col * ES);
-          g2[j].load(gs + (half + col) * ES);
+        for (int j = 0; j < NP; ++j) {
+          const int r = r0 + j * L.rpw;
+          x1[j].w = x2[j].w = g1[j].w = g2[j].w = u32x4{0u, 0u, 0u, 0u};
+          if (r < rows) {
+            x1[j].load(xs + r * xh + col * ES);
+            x2[j].load(xs + r * xh + (half + col) * ES);
+            g1[j].load(gs + r * gh + col * ES);
+            g2[j].load(gs + r * gh + (half + col) * ES);
+          }
         }
-      }
 #pragma unroll
-      for (int j = 0; j < kBwdPasses; ++j) {
-        if (inside) {
+        for (int j = 0; j < NP; ++j) {
+          const int r = r0 + j * L.rpw;
+          const bool live = r < rows;
+          if (!inside) {  // (the same for every lane)
+            if (live) {
+              g1[j].store(os + r * oh + col * ES);
+              g2[j].store(os + r * oh + (half + col) * ES);
+            }
+            continue;
+          }
           // g' = R(-angle) dy (the transpose of the forward rotation)
+          Ch y1, y2;
+          float ss = 0.f, tw = 0.f;
 #pragma unroll
           for (int e = 0; e < EPL; ++e) {
-            const float a = g1[j].v[e], bq = g2[j].v[e];
-            g1[j].v[e] = add_rn(mul_rn(a, c[e]), mul_rn(bq, s[e]));
-            g2[j].v[e] = add_rn(mul_rn(bq, c[e]), mul_rn(-a, s[e]));
+            const float a = g1[j].get(e), b = g2[j].get(e);
+            const float u = x1[j].get(e), v = x2[j].get(e);
+            y1.v[e] = add_rn(mul_rn(a, c[e]), mul_rn(b, s[e]));
+            y2.v[e] = add_rn(mul_rn(b, c[e]), mul_rn(-a, s[e]));
+            ss += u * u + v * v;
+            tw += u * wsh[side][col + e] * y1.v[e] + v * wsh[side][half + col + e] * y2.v[e];
           }
-          float ss = 0.f, tw = 0.f;
-          if (dst[j]) {
-#pragma unroll
-            for (int e = 0; e < EPL; ++e) {
-              const float w1 = isq[j] ? wq1[e] : wk1[e], w2 = isq[j] ? wq2[e] : wk2[e];
-              ss += x1[j].v[e] * x1[j].v[e] + x2[j].v[e] * x2[j].v[e];
-              tw += x1[j].v[e] * w1 * g1[j].v[e] + x2[j].v[e] * w2 * g2[j].v[e];
-            }
-          }
+          // (a lane past the rows holds zeros; every lane joins the sums)
           ss = row_sum(ss, L.lpr);
           tw = row_sum(tw, L.lpr);
-          const bool has_w = isq[j] ? P.wq != nullptr : P.wk != nullptr;
-          if (dst[j] && has_w) {
+          if (has_w) {
             const float rr = rsqrtf(ss * inv_d + P.eps);
             const float k3 = rr * rr * rr * tw * inv_d;
+            if (live) {
 #pragma unroll
-            for (int e = 0; e < EPL; ++e) {
-              const float w1 = isq[j] ? wq1[e] : wk1[e], w2 = isq[j] ? wq2[e] : wk2[e];
-              const float xr1 = x1[j].v[e] * rr, xr2 = x2[j].v[e] * rr;
-              if (isq[j]) aq1[e] += xr1 * g1[j].v[e], aq2[e] += xr2 * g2[j].v[e];
-              else ak1[e] += xr1 * g1[j].v[e], ak2[e] += xr2 * g2[j].v[e];
-              g1[j].v[e] = rr * w1 * g1[j].v[e] - x1[j].v[e] * k3;
-              g2[j].v[e] = rr * w2 * g2[j].v[e] - x2[j].v[e] * k3;
+              for (int e = 0; e < EPL; ++e) {
+                const float u = x1[j].get(e), v = x2[j].get(e);
+                dw1[side][e] += u * rr * y1.v[e];
+                dw2[side][e] += v * rr * y2.v[e];
+                y1.v[e] = rr * wsh[side][col + e] * y1.v[e] - u * k3;
+                y2.v[e] = rr * wsh[side][half + col + e] * y2.v[e] - v * k3;
+              }
             }
           }
-        }
-        if (dst[j]) {
-          g1[j].store(dst[j] + col * ES);
-          g2[j].store(dst[j] + (half + col) * ES);
+          if (live) {
+            y1.store(os + r * oh + col * ES);
+            y2.store(os + r * oh + (half + col) * ES);
+          }
         }
       }
-    }
+    });
   }
 
   // dw partials: lanes sharing columns (lane % lpr), then the waves, in a
@@ -407,19 +448,21 @@ __global__ __launch_bounds__(64 * kRopeWaves) void rope_norm_bwd_kernel(const Ro
 #pragma unroll
   for (int e = 0; e < EPL; ++e) {
     for (int m = L.lpr; m < 64; m <<= 1) {
-      aq1[e] += __shfl_xor(aq1[e], m);
-      aq2[e] += __shfl_xor(aq2[e], m);
-      ak1[e] += __shfl_xor(ak1[e], m);
-      ak2[e] += __shfl_xor(ak2[e], m);
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        dw1[side][e] += __shfl_xor(dw1[side][e], m);
+        dw2[side][e] += __shfl_xor(dw2[side][e], m);
+      }
     }
   }
   if (lane < L.lpr) {
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
-      red[0][wv][col + e] = aq1[e];
-      red[0][wv][half + col + e] = aq2[e];
-      red[1][wv][col + e] = ak1[e];
-      red[1][wv][half + col + e] = ak2[e];
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        red[side][wv][col + e] = dw1[side][e];
+        red[side][wv][half + col + e] = dw2[side][e];
+      }
     }
   }
   __syncthreads();
@@ -467,10 +510,21 @@ __global__ __launch_bounds__(1024) void rope_dw_reduce_kernel(const RopeParams P
 
 }  // namespace
 
-int rope_blocks(int T) {
-  const int per_block = kRopeWaves * kRopeTokensPerWave;
-  return (T + per_block - 1) / per_block;
+// Consecutive tokens per wave.  A wave's tokens are one chain of latencies
+// and share its start (and, in the norm backward, its dw partials): few of
+// them while the waves leave the chip with room, four once they fill it.
+// us with 1 / 2 / 4 tokens (bf16, d = 128, 32 heads), norm + RoPE forward: 400
+// tokens x 16 heads 7.5 / 9.1 / 15.3, 4000 tokens 15.7 / 19.6 / 26.3, 16384
+// 53.8 / 52.9 / 49.5; norm backward 12.3 / 13.6 / 18.9, 28.9 / 26.8 / 34.5,
+// 94.7 / 91.9 / 89.0 (fp32, 6000 tokens: forward 37 / 35 / 46, backward 59 /
+// 57 / 66).
+static int fwd_tokens_per_wave(int T) { return T <= 4096 ? 1 : T <= 12288 ? 2 : 4; }
+static int bwd_tokens_per_wave(int T) { return T <= 1024 ? 1 : T <= 12288 ? 2 : 4; }
+static int blocks_of(int T, int tpw) {
+  return (int)(((int64_t)T + kRopeWaves * tpw - 1) / (kRopeWaves * tpw));
 }
+
+int rope_bwd_blocks(int T) { return blocks_of(T, bwd_tokens_per_wave(T)); }
 
 namespace {
 template <int DT>
@@ -482,9 +536,11 @@ void launch_rope_dt(const RopeParams& P, dim3 grid, dim3 block, hipStream_t s) {
 }
 }  // namespace
 
-hipError_t launch_rope(const RopeParams& P, hipStream_t s) {
+hipError_t launch_rope(const RopeParams& args, hipStream_t s) {
+  RopeParams P = args;
   if (P.T <= 0 || P.Hq + P.Hk <= 0) return hipSuccess;
-  const dim3 grid(rope_blocks(P.T)), block(64 * kRopeWaves);
+  P.tpw = fwd_tokens_per_wave(P.T);
+  const dim3 grid(blocks_of(P.T, P.tpw)), block(64 * kRopeWaves);
   switch (P.dtype) {
     case kRopeBF16: launch_rope_dt<kRopeBF16>(P, grid, block, s); break;
     case kRopeF16: launch_rope_dt<kRopeF16>(P, grid, block, s); break;
@@ -494,9 +550,11 @@ hipError_t launch_rope(const RopeParams& P, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_rope_norm_bwd(const RopeParams& P, hipStream_t s) {
+hipError_t launch_rope_norm_bwd(const RopeParams& args, hipStream_t s) {
+  RopeParams P = args;
   if (P.T <= 0 || P.Hq + P.Hk <= 0) return hipSuccess;
-  const int nb = rope_blocks(P.T);
+  P.tpw = bwd_tokens_per_wave(P.T);
+  const int nb = rope_bwd_blocks(P.T);
   const dim3 grid(nb), block(64 * kRopeWaves);
   switch (P.dtype) {
     case kRopeBF16: hipLaunchKernelGGL(rope_norm_bwd_kernel<kRopeBF16>, grid, block, 0, s, P); break;
