@@ -77,14 +77,19 @@ __device__ void zero_uncovered_rows(const BwdParams& P, int w, int nw) {
   }
 }
 
-template <int D, int RPL, bool F16>
+// NG (key groups): with few tiles, NG groups of 4 waves share a tile, group g
+// taking key steps g, g + NG, ... with a ring of its own, as in the forward;
+// the groups' accumulators are summed in group 0 through the idle ring.
+template <int D, int RPL, bool F16, int NG>
 __device__ __forceinline__ void dq_body(const BwdParams& P) {
   using C = DqCfg<D, RPL>;
-  __shared__ __attribute__((aligned(1024))) uint8_t st0[C::STAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t st1[C::STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t st0[NG * C::STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t st1[NG * C::STAGE];
   const Problem& p = P.p;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wv = uni(tid >> 6);
+  const int wave = uni(tid >> 6);
+  const int wv = NG > 1 ? wave & 3 : wave;  // wave within its key group
+  const int grp = NG > 1 ? wave >> 2 : 0;
   const int l32 = lane & 31, hl = lane >> 5;
   const int h = blockIdx.x % p.H;
   const int tix = blockIdx.x / p.H;
@@ -132,6 +137,9 @@ __device__ __forceinline__ void dq_body(const BwdParams& P) {
   int kv_hi = e.lk;
   if (p.causal) kv_hi = min(kv_hi, min(e.lq, q0 + C::BM));
   const int nkb = cdiv(max(kv_hi, 0), C::BN);
+  // this group's ring
+  uint8_t* const ring0 = NG > 1 ? st0 + grp * C::STAGE : st0;
+  uint8_t* const ring1 = NG > 1 ? st1 + grp * C::STAGE : st1;
 
   const uint32_t krb = (uint32_t)P.k.ss * 2u, vrb = (uint32_t)P.v.ss * 2u;
   const uint32_t rkrb = (uint32_t)P.rk.ss * 2u;
@@ -155,7 +163,7 @@ __device__ __forceinline__ void dq_body(const BwdParams& P) {
 
   // The first key tile's DMA goes out before the row loads below, so the
   // two latencies overlap instead of adding up.
-  if (nkb > 0) issue(0, st0);
+  if (grp < nkb) issue(grp, ring0);
   __builtin_amdgcn_sched_barrier(0);
 
   // Stationary B operands: Qa and dO rows of this lane's query.
@@ -239,10 +247,11 @@ __device__ __forceinline__ void dq_body(const BwdParams& P) {
 
   auto step = [&](int it, const uint8_t* cur, uint8_t* nxt) {
     ring_barrier<0>();
-    if (it + 1 < nkb) issue(it + 1, nxt);
+    if (it + NG < nkb) issue(it + NG, nxt);
     __builtin_amdgcn_sched_barrier(0);
     const int kbase = it * C::BN;
-    const bool active = (wq0 <= wq_last) && (!p.causal || kbase <= wq_last);
+    const bool active =
+        (wq0 <= wq_last) && (!p.causal || kbase <= wq_last) && (NG == 1 || it < nkb);
     if (!active) return;
     const bool diag = p.causal && kbase + C::BN - 1 > wq0;
     const uint8_t* kt = cur;
@@ -385,9 +394,47 @@ __device__ __forceinline__ void dq_body(const BwdParams& P) {
       }
   };
 
-  for (int it = 0; it < nkb; it += 2) {
-    step(it, st0, st1);
-    if (it + 1 < nkb) step(it + 1, st1, st0);
+  // (every group makes the same number of steps: they share the barriers)
+  for (int it = 0; it < nkb; it += 2 * NG) {
+    step(it + grp, ring0, ring1);
+    if (it + NG < nkb) step(it + NG + grp, ring1, ring0);
+  }
+
+  if constexpr (NG > 1) {
+    // Sum the groups' accumulators in group 0, wave by wave, the head-dim
+    // part and then the rank part (as they lie in the registers, 16 bytes
+    // per lane).
+    constexpr int HAND = 32 * D * 4;
+    static_assert(2 * HAND <= NG * C::STAGE && RPL <= D, "two waves' hand-over fits in a stage");
+    float* hand = (float*)((wv < 2 ? st0 : st1) + (wv & 1) * HAND);
+    static_for<C::NRB ? 2 : 1>([&](auto part_) {
+      constexpr int A0 = decltype(part_)::value ? C::NDB : 0;
+      constexpr int A1 = decltype(part_)::value ? C::NDB + C::NRB : C::NDB;
+      for (int j = 1; j < NG; ++j) {
+        __syncthreads();  // the ring (or the last hand-over) has been read
+        if (grp == j) {
+#pragma unroll
+          for (int f = A0; f < A1; ++f)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              *(f32x4_t*)(hand + (((f - A0) * 4 + i) * 64 + lane) * 4) =
+                  f32x4_t{acc[f][4 * i], acc[f][4 * i + 1], acc[f][4 * i + 2], acc[f][4 * i + 3]};
+        }
+        __syncthreads();
+        if (grp == 0) {
+#pragma unroll
+          for (int f = A0; f < A1; ++f)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const f32x4_t x = *(const f32x4_t*)(hand + (((f - A0) * 4 + i) * 64 + lane) * 4);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[f][4 * i + e] += x[e];
+            }
+        }
+      }
+    });
+    __syncthreads();
+    if (grp != 0) return;
   }
 
   // The loop accumulated dS = P (dP - delta); dA = c dS.  This lane's part
@@ -434,7 +481,7 @@ __device__ __forceinline__ void dq_body(const BwdParams& P) {
   // half w % 2) and stores them as whole rows, 16 bytes per lane.
   using QS = RowStage<D>;
   static_assert(2 * QS::BYTES <= C::STAGE, "the epilogue staging fits in a ring stage");
-  __syncthreads();
+  if constexpr (NG == 1) __syncthreads();
   uint8_t* obuf = (wv < 2 ? st0 : st1) + (wv & 1) * QS::BYTES;
   const int nrows = max(min(32, e.lq - wq0), 0);
   const float sq = p.qa * p.c;
@@ -483,15 +530,17 @@ __device__ __forceinline__ void dq_body(const BwdParams& P) {
   }
 }
 
-// WAVES: waves per SIMD the register budget is cut for.
-#define FNA2_DQ_KERNEL(D, RPL, WAVES)                                                    \
-  __global__ __launch_bounds__(256, WAVES) void dq_kernel_d##D##_r##RPL(const BwdParams P) { \
-    dq_body<D, RPL, false>(P);                                                           \
-  }                                                                                      \
-  __global__ __launch_bounds__(256, WAVES) void dq_kernel_d##D##_r##RPL##_f16(             \
-      const BwdParams P) {                                                               \
-    dq_body<D, RPL, true>(P);                                                            \
+// WAVES: waves per SIMD the register budget is cut for; _kg: with as many key
+// groups, which fill a CU with one workgroup.
+#define FNA2_DQ_ONE(NAME, D, RPL, F16, NG, WAVES)                                \
+  __global__ __launch_bounds__(256 * NG, WAVES) void NAME(const BwdParams P) {   \
+    dq_body<D, RPL, F16, NG>(P);                                                 \
   }
+#define FNA2_DQ_KERNEL(D, RPL, WAVES)                                            \
+  FNA2_DQ_ONE(dq_kernel_d##D##_r##RPL, D, RPL, false, 1, WAVES)                  \
+  FNA2_DQ_ONE(dq_kernel_d##D##_r##RPL##_f16, D, RPL, true, 1, WAVES)             \
+  FNA2_DQ_ONE(dq_kernel_d##D##_r##RPL##_kg, D, RPL, false, WAVES, WAVES)         \
+  FNA2_DQ_ONE(dq_kernel_d##D##_r##RPL##_f16_kg, D, RPL, true, WAVES, WAVES)
 FNA2_DQ_KERNEL(64, 0, 3)
 FNA2_DQ_KERNEL(64, 32, 3)
 FNA2_DQ_KERNEL(64, 64, 2)
@@ -499,24 +548,27 @@ FNA2_DQ_KERNEL(128, 0, 2)
 FNA2_DQ_KERNEL(128, 32, 2)
 FNA2_DQ_KERNEL(128, 64, 2)
 #undef FNA2_DQ_KERNEL
+#undef FNA2_DQ_ONE
 
 }  // namespace
+
+int dq_key_groups(int D, int rpl) { return D == 64 && rpl <= 32 ? 3 : 2; }
 
 hipError_t launch_bwd_dq(const BwdParams& P, int rpl, int grid, hipStream_t s) {
   if (grid <= 0) return hipSuccess;
   void (*k)(const BwdParams) = nullptr;
-  if (P.p.f16) {
-    if (P.p.D == 64)
-      k = rpl == 0 ? dq_kernel_d64_r0_f16 : rpl == 32 ? dq_kernel_d64_r32_f16 : dq_kernel_d64_r64_f16;
-    if (P.p.D == 128)
-      k = rpl == 0 ? dq_kernel_d128_r0_f16 : rpl == 32 ? dq_kernel_d128_r32_f16 : dq_kernel_d128_r64_f16;
-  } else {
-    if (P.p.D == 64) k = rpl == 0 ? dq_kernel_d64_r0 : rpl == 32 ? dq_kernel_d64_r32 : dq_kernel_d64_r64;
-    if (P.p.D == 128)
-      k = rpl == 0 ? dq_kernel_d128_r0 : rpl == 32 ? dq_kernel_d128_r32 : dq_kernel_d128_r64;
-  }
+  const bool f16 = P.p.f16 != 0, kg = P.key_groups > 1;
+#define FNA2_DQ_OF(D, RPL)                                                     \
+  (f16 ? (kg ? dq_kernel_d##D##_r##RPL##_f16_kg : dq_kernel_d##D##_r##RPL##_f16) \
+       : (kg ? dq_kernel_d##D##_r##RPL##_kg : dq_kernel_d##D##_r##RPL))
+  if (P.p.D == 64)
+    k = rpl == 0 ? FNA2_DQ_OF(64, 0) : rpl == 32 ? FNA2_DQ_OF(64, 32) : FNA2_DQ_OF(64, 64);
+  if (P.p.D == 128)
+    k = rpl == 0 ? FNA2_DQ_OF(128, 0) : rpl == 32 ? FNA2_DQ_OF(128, 32) : FNA2_DQ_OF(128, 64);
+#undef FNA2_DQ_OF
   if (!k || (rpl != 0 && rpl != 32 && rpl != 64)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, s, P);
+  const int threads = 256 * (kg ? dq_key_groups(P.p.D, rpl) : 1);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(threads), 0, s, P);
   return hipGetLastError();
 }
 

@@ -161,6 +161,36 @@ BwdWs bwd_ws(const fna2_problem& p) {
   return w;
 }
 
+// Whether the forward's / dQ's query tiles are so few that the key groups'
+// variants (one workgroup of 8 to 16 waves per tile and CU) are the faster:
+// the tiles' longest key loop is then the kernel's time, and the groups cut
+// it, for some 3 us of combining.  That takes `min_keys` keys in the longest
+// tile, and at most one tile per CU -- two under the causal mask, whose tiles
+// differ in length.  Measured, us without -> with key groups, H heads x S:
+//   forward d64 r16  8x512 15.4 -> 15.3, 8x1024 23.8 -> 19.9, 16x2048 39.2 ->
+//     30.4, 16x4096 (512 tiles) 72.5 -> 59.7, non-causal 32x2048 (512) 54 -> 57,
+//     32x3001 (768) 62 -> 73
+//   forward d128 r32 8x256 14.8 -> 15.4, 8x512 21.3 -> 19.2, 16x2048 61 -> 43,
+//     32x1531 (384) 48.6 -> 39.5, 32x3001 (768) 101 -> 108
+//   dQ d64 r16  8x512 21.4 -> 20.9, 8x1024 34.2 -> 27.7, 16x2048 58.8 -> 41.9,
+//     32x2048 (512) 60 -> 55, non-causal 75 -> 82
+//   dQ d128 r32  8x512 25.8 -> 25.7, 8x1024 39.7 -> 36.5, 16x2048 69 -> 60,
+//     32x1531 (384) 58.6 -> 54.2, 32x3001 (768) 135 -> 154
+// (A varlen call counts its tiles by the tokens and half a tile per sequence
+// and takes the hinted length.)
+constexpr int kSplitCUs = 256;  // (a fixed figure: the answer depends on the arguments alone)
+bool few_tiles(const fna2_problem& p, int64_t min_keys) {
+  int64_t tiles, keys;
+  if (p.varlen) {
+    tiles = cdiv64(p.total_q, kFwdBM) + p.batch / 2;
+    keys = p.seqlen_k > 0 ? std::min(p.seqlen_k, p.total_k) : p.total_k / std::max(p.batch, 1);
+  } else {
+    tiles = (int64_t)p.batch * cdiv64(p.seqlen_q, kFwdBM);
+    keys = p.causal ? std::min(p.seqlen_q, p.seqlen_k) : p.seqlen_k;
+  }
+  return tiles * p.heads <= kSplitCUs * (p.causal ? 2 : 1) && keys >= min_keys;
+}
+
 // dK/dV items in chunks.  The persistent dK/dV kernel deals (key tile, KV
 // head) items to the CUs; where these are fewer than the CUs, or one item is
 // longer than a CU's share of the work, the time is the longest item's.
@@ -184,7 +214,6 @@ struct KvSplit {
   int64_t tiles = 0;
   size_t kv_part = 0, drk_part = 0, bytes = 0;  // offsets in the split's own region
 };
-constexpr int kSplitCUs = 256;  // (a fixed figure: the size depends on the arguments alone)
 constexpr int64_t kSplitMaxBytes = (int64_t)512 << 20;
 
 KvSplit kv_split(const fna2_problem& p) {
@@ -564,6 +593,9 @@ int fwd_launch(const fna2_fwd_args* a, void* ws, hipStream_t stream) {
   }
   const int rpl = fna2::padded_rank32(K.p.H_G, K.p.R);
   if (!mark(a->events, 0, stream)) return FNA2_E_LAUNCH;
+  K.key_groups = few_tiles(p, p.head_dim == 128 ? 512 : 768)
+                     ? fna2::fwd_key_groups(p.head_dim, rpl)
+                     : 1;
   if (fna2::launch_fwd(K, rpl, (int)g.fwd_grid, stream) != hipSuccess) return FNA2_E_LAUNCH;
   if (!mark(a->events, 1, stream)) return FNA2_E_LAUNCH;
   return FNA2_OK;
@@ -696,6 +728,7 @@ int fna2_bwd(const fna2_bwd_args* a, void* stream_ptr) {
     // (with a plan, one more row of workgroups than tiles can fill, so that
     // spare workgroups exist for the zeroing whatever the lengths)
     const int dq_grid = (int)g.dq_grid + (K.zero_uncovered ? p.heads : 0);
+    K.key_groups = few_tiles(p, 768) ? fna2::dq_key_groups(p.head_dim, rpl) : 1;
     if (rows_q(p) > 0 && fna2::launch_bwd_dq(K, rpl, dq_grid, stream) != hipSuccess)
       return FNA2_E_LAUNCH;
     if (!mark(a->events, 1, stream) || !mark(a->events, 2, stream)) return FNA2_E_LAUNCH;

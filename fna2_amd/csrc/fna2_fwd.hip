@@ -58,17 +58,25 @@ struct FwdCfg {
 // score tile needs no scaling by b -- 16 VALU multiplies fewer per 32 x 32
 // tile for one more MFMA, and no register more (the halves are the padding
 // of the rank tile).
-template <int D, int RPL, bool F16, bool S16>
+//
+// NG (key groups): with few tiles, NG groups of 4 waves share a tile, group g
+// taking key steps g, g + NG, ... with a ring of its own; at the end the
+// groups' (O, m, l) are combined in group 0 through the idle ring.  The
+// key loop, which is the kernel's time while the grid does not fill the
+// chip, is then NG times shorter.
+template <int D, int RPL, bool F16, bool S16, int NG>
 __device__ __forceinline__ void fwd_body(const FwdParams& P) {
   using C = FwdCfg<D, RPL>;
   static_assert(!S16 || RPL == 32, "the split uses the padding of a 32-wide rank tile");
   // Two stages as separate objects: the compiler can then tell that reads of
   // one stage never alias the DMA into the other and does not wait for it.
-  __shared__ __attribute__((aligned(1024))) uint8_t stage0[C::STAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t stage1[C::STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t stage0[NG * C::STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t stage1[NG * C::STAGE];
   const Problem& p = P.p;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (scalar)
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (scalar)
+  const int wv = NG > 1 ? wave & 3 : wave;                     // wave within its key group
+  const int grp = NG > 1 ? wave >> 2 : 0;
   const int l32 = lane & 31, hl = lane >> 5;
   const int h = blockIdx.x % p.H;
   const int tix = blockIdx.x / p.H;
@@ -106,6 +114,9 @@ __device__ __forceinline__ void fwd_body(const FwdParams& P) {
   int kv_hi = e.lk;
   if (p.causal) kv_hi = min(kv_hi, min(e.lq, q0 + C::BM));
   const int nkv = cdiv(max(kv_hi, 0), C::BN);
+  // this group's ring
+  uint8_t* const ring0 = NG > 1 ? stage0 + grp * C::STAGE : stage0;
+  uint8_t* const ring1 = NG > 1 ? stage1 + grp * C::STAGE : stage1;
 
   // DMA plans (lane offsets are tile-invariant; descriptors move per tile).
   const uint32_t krb = (uint32_t)P.k.ss * 2u, vrb = (uint32_t)P.v.ss * 2u;
@@ -135,7 +146,7 @@ __device__ __forceinline__ void fwd_body(const FwdParams& P) {
 
   // The first key tile's DMA goes out before the query loads below, so the
   // two latencies overlap instead of adding up.
-  if (nkv > 0) issue(0, stage0);
+  if (grp < nkv) issue(grp, ring0);
   __builtin_amdgcn_sched_barrier(0);
 
   // Query operand (B of S^T): lane holds Qa[qrow][16s + 8hl .. +7].
@@ -202,10 +213,11 @@ __device__ __forceinline__ void fwd_body(const FwdParams& P) {
   // then compute on this one.
   auto step = [&](int kt, const uint8_t* cur, uint8_t* nxt) {
     ring_barrier<0>();
-    if (kt + 1 < nkv) issue(kt + 1, nxt);
+    if (kt + NG < nkv) issue(kt + NG, nxt);
     __builtin_amdgcn_sched_barrier(0);  // keep the whole prefetch ahead of the compute
     const int kbase = kt * C::BN;
-    const bool active = (wq0 <= wq_last) && (!p.causal || kbase <= wq_last);
+    const bool active =
+        (wq0 <= wq_last) && (!p.causal || kbase <= wq_last) && (NG == 1 || kt < nkv);
     if (!active) return;
     const uint8_t* kl = cur;
     const uint8_t* rl = kl + C::KBYTES;
@@ -320,9 +332,51 @@ __device__ __forceinline__ void fwd_body(const FwdParams& P) {
     }
   };
 
-  for (int kt = 0; kt < nkv; kt += 2) {
-    step(kt, stage0, stage1);
-    if (kt + 1 < nkv) step(kt + 1, stage1, stage0);
+  // (every group makes the same number of steps: they share the barriers)
+  for (int kt = 0; kt < nkv; kt += 2 * NG) {
+    step(kt + grp, ring0, ring1);
+    if (kt + NG < nkv) step(kt + NG + grp, ring1, ring0);
+  }
+
+  if constexpr (NG > 1) {
+    // Combine the groups: group j hands over its accumulators as they lie in
+    // the registers (16 bytes per lane), its running maximum and sum (per
+    // lane half, under a maximum both halves share), wave by wave.
+    constexpr int OB = 32 * D * 4, HAND = OB + 512;
+    static_assert(2 * HAND <= NG * C::STAGE, "two waves' hand-over fits in a stage");
+    float* hand = (float*)((wv < 2 ? stage0 : stage1) + (wv & 1) * HAND);
+    for (int j = 1; j < NG; ++j) {
+      __syncthreads();  // the ring (or the last hand-over) has been read
+      if (grp == j) {
+#pragma unroll
+        for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            *(f32x4_t*)(hand + ((d * 4 + i) * 64 + lane) * 4) =
+                f32x4_t{oacc[d][4 * i], oacc[d][4 * i + 1], oacc[d][4 * i + 2], oacc[d][4 * i + 3]};
+        *(f32x2*)(hand + OB / 4 + 2 * lane) = f32x2{m_i, l_i};
+      }
+      __syncthreads();
+      if (grp == 0) {
+        const f32x2 ml = *(const f32x2*)(hand + OB / 4 + 2 * lane);
+        const float m_new = fmaxf(m_i, ml[0]);
+        const float ref = m_new == kNegInf ? 0.f : m_new;
+        const float wa = __builtin_amdgcn_exp2f((m_i - ref) * p.c2);  // (-inf: 0)
+        const float wb = __builtin_amdgcn_exp2f((ml[0] - ref) * p.c2);
+        m_i = m_new;
+        l_i = l_i * wa + ml[1] * wb;
+#pragma unroll
+        for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const f32x4_t o = *(const f32x4_t*)(hand + ((d * 4 + i) * 64 + lane) * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) oacc[d][4 * i + e] = oacc[d][4 * i + e] * wa + o[e] * wb;
+          }
+      }
+    }
+    __syncthreads();
+    if (grp != 0) return;
   }
 
   const float l_tot = wave_pair_sum(l_i);
@@ -335,7 +389,7 @@ __device__ __forceinline__ void fwd_body(const FwdParams& P) {
     // c3's forward 90 -> 83 us).
     using OS = RowStage<D>;
     static_assert(2 * OS::BYTES <= C::STAGE, "the epilogue staging fits in a ring stage");
-    __syncthreads();
+    if constexpr (NG == 1) __syncthreads();
     uint8_t* obuf = (wv < 2 ? stage0 : stage1) + (wv & 1) * OS::BYTES;
 #pragma unroll
     for (int d = 0; d < D / 32; ++d)
@@ -369,46 +423,48 @@ __device__ __forceinline__ void fwd_body(const FwdParams& P) {
 
 // One non-template kernel per (D, padded rank, element type): every kernel
 // gets its own host launch stub.  WAVES: waves per SIMD the register budget
-// is cut for.
-#define FNA2_FWD_KERNEL(D, RNAME, RPL, S16, WAVES)                                          \
-  __global__ __launch_bounds__(256, WAVES) void fwd_kernel_d##D##_r##RNAME(const FwdParams P) { \
-    fwd_body<D, RPL, false, S16>(P);                                                         \
-  }                                                                                          \
-  __global__ __launch_bounds__(256, WAVES) void fwd_kernel_d##D##_r##RNAME##_f16(              \
-      const FwdParams P) {                                                                   \
-    fwd_body<D, RPL, true, S16>(P);                                                          \
+// is cut for; _kg: with the key groups that fill a CU with one workgroup.
+#define FNA2_FWD_ONE(NAME, D, RPL, F16, S16, NG, WAVES)                              \
+  __global__ __launch_bounds__(256 * NG, WAVES) void NAME(const FwdParams P) {       \
+    fwd_body<D, RPL, F16, S16, NG>(P);                                               \
   }
-FNA2_FWD_KERNEL(64, 0, 0, false, 2)
-FNA2_FWD_KERNEL(64, 16, 32, true, 2)
-FNA2_FWD_KERNEL(64, 32, 32, false, 2)
-FNA2_FWD_KERNEL(64, 64, 64, false, 2)
-FNA2_FWD_KERNEL(128, 0, 0, false, 3)
-FNA2_FWD_KERNEL(128, 32, 32, false, 3)
-FNA2_FWD_KERNEL(128, 64, 64, false, 3)
+#define FNA2_FWD_KERNEL(D, RNAME, RPL, S16, WAVES, NG)                               \
+  FNA2_FWD_ONE(fwd_kernel_d##D##_r##RNAME, D, RPL, false, S16, 1, WAVES)             \
+  FNA2_FWD_ONE(fwd_kernel_d##D##_r##RNAME##_f16, D, RPL, true, S16, 1, WAVES)        \
+  FNA2_FWD_ONE(fwd_kernel_d##D##_r##RNAME##_kg, D, RPL, false, S16, NG, NG)          \
+  FNA2_FWD_ONE(fwd_kernel_d##D##_r##RNAME##_f16_kg, D, RPL, true, S16, NG, NG)
+FNA2_FWD_KERNEL(64, 0, 0, false, 2, 4)
+FNA2_FWD_KERNEL(64, 16, 32, true, 2, 4)
+FNA2_FWD_KERNEL(64, 32, 32, false, 2, 4)
+FNA2_FWD_KERNEL(64, 64, 64, false, 2, 3)
+FNA2_FWD_KERNEL(128, 0, 0, false, 3, 3)
+FNA2_FWD_KERNEL(128, 32, 32, false, 3, 3)
+FNA2_FWD_KERNEL(128, 64, 64, false, 3, 3)
 #undef FNA2_FWD_KERNEL
+#undef FNA2_FWD_ONE
 
 }  // namespace
+
+int fwd_key_groups(int D, int rpl) { return D == 64 && rpl <= 32 ? 4 : 3; }
 
 hipError_t launch_fwd(const FwdParams& P, int rpl, int grid, hipStream_t s) {
   if (grid <= 0) return hipSuccess;
   void (*k)(const FwdParams) = nullptr;
   // d = 64 with R <= 16: the split rank operand (S16)
   const bool r16 = rpl == 32 && P.p.R <= 16;
-  if (P.p.f16) {
-    if (P.p.D == 64)
-      k = rpl == 0 ? fwd_kernel_d64_r0_f16
-          : rpl == 32 ? (r16 ? fwd_kernel_d64_r16_f16 : fwd_kernel_d64_r32_f16)
-                      : fwd_kernel_d64_r64_f16;
-    if (P.p.D == 128)
-      k = rpl == 0 ? fwd_kernel_d128_r0_f16 : rpl == 32 ? fwd_kernel_d128_r32_f16 : fwd_kernel_d128_r64_f16;
-  } else {
-    if (P.p.D == 64)
-      k = rpl == 0 ? fwd_kernel_d64_r0
-          : rpl == 32 ? (r16 ? fwd_kernel_d64_r16 : fwd_kernel_d64_r32) : fwd_kernel_d64_r64;
-    if (P.p.D == 128) k = rpl == 0 ? fwd_kernel_d128_r0 : rpl == 32 ? fwd_kernel_d128_r32 : fwd_kernel_d128_r64;
-  }
+  const bool f16 = P.p.f16 != 0, kg = P.key_groups > 1;
+#define FNA2_FWD_OF(D, RNAME)                                                          \
+  (f16 ? (kg ? fwd_kernel_d##D##_r##RNAME##_f16_kg : fwd_kernel_d##D##_r##RNAME##_f16) \
+       : (kg ? fwd_kernel_d##D##_r##RNAME##_kg : fwd_kernel_d##D##_r##RNAME))
+  if (P.p.D == 64)
+    k = rpl == 0 ? FNA2_FWD_OF(64, 0)
+        : rpl == 32 ? (r16 ? FNA2_FWD_OF(64, 16) : FNA2_FWD_OF(64, 32)) : FNA2_FWD_OF(64, 64);
+  if (P.p.D == 128)
+    k = rpl == 0 ? FNA2_FWD_OF(128, 0) : rpl == 32 ? FNA2_FWD_OF(128, 32) : FNA2_FWD_OF(128, 64);
+#undef FNA2_FWD_OF
   if (!k || (rpl != 0 && rpl != 32 && rpl != 64)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, s, P);
+  const int threads = 256 * (kg ? fwd_key_groups(P.p.D, rpl) : 1);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(threads), 0, s, P);
   return hipGetLastError();
 }
 

@@ -11,6 +11,7 @@ struct FwdParams {
   const float* gs;
   const TileRec* tiles;  // varlen: device tile list (null in dense mode)
   const int* n_tiles;  // varlen: device tile count
+  int key_groups;      // > 1: groups of waves share a tile's keys (fwd_key_groups)
 };
 
 struct BwdParams {
@@ -32,6 +33,7 @@ struct BwdParams {
   int split_tiles, split_log2;
   float* kv_part;   // [split_tiles][H_KV][2^split_log2] slots of dK | dV
   float* drk_part;  // [split_tiles][H_KV][drk_slots] slots of dRk
+  int key_groups;  // dQ kernel, > 1: as in the forward (dq_key_groups)
   int zero_uncovered;  // varlen: the dQ kernel's spare workgroups zero the
                        // gradient rows of tokens outside every sequence
 };
@@ -142,6 +144,9 @@ int decode_stage_bytes(int D, int rc);
 hipError_t launch_decode(const DecodeParams& P, int rc, hipStream_t s);
 hipError_t launch_decode_merge(const DecodeParams& P, hipStream_t s);
 
+// Key groups of the forward and dQ kernels' _kg variants.
+int fwd_key_groups(int D, int rpl);
+int dq_key_groups(int D, int rpl);
 hipError_t launch_fwd(const FwdParams& P, int rp, int grid, hipStream_t s);
 hipError_t launch_bwd_dkdv(const BwdParams& P, int rpl, int grid, hipStream_t s);
 hipError_t launch_bwd_dq(const BwdParams& P, int rpl, int grid, hipStream_t s);
