@@ -150,7 +150,7 @@ __device__ __forceinline__ void dq_body(const BwdParams& P) {
   if constexpr (RPL > 0) dr.init(wv, lane, rkrb, p.R / 8);
   auto issue = [&](int it, uint8_t* st) {
     const int k0 = it * C::BN;
-    const uint32_t rows = (uint32_t)max(min(C::BN, e.lk - k0), 0);
+    const uint32_t rows = (uint32_t)clamp_rows(e.lk - k0, C::BN);
     dk.issue(make_rsrc(kb + (int64_t)k0 * P.k.ss, rows * krb), st, wv);
     if constexpr (RPL > 0) {
       // (RANK_ALL: a vanilla head's rank tile is a zero-size range, so the

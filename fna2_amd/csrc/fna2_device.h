@@ -95,6 +95,16 @@ __device__ __forceinline__ float here_s(float x) {
   return x;
 }
 
+// A wave-uniform int, opaque where it is used.  clamp_rows: min(max(x, 0),
+// hi) of a uniform x in scalar instructions; the compiler would make it one
+// v_med3 and the products of it vector multiplies, each read back by
+// v_readfirstlane, in the key loops' address path.
+__device__ __forceinline__ int here_i(int x) {
+  asm volatile("" : "+s"(x));
+  return x;
+}
+__device__ __forceinline__ int clamp_rows(int x, int hi) { return max(here_i(min(uni(x), hi)), 0); }
+
 // Extents of sequence b (b may differ per lane).
 __device__ __forceinline__ SeqExt seq_ext(const Problem& p, int b) {
   SeqExt e;
@@ -273,11 +283,23 @@ __device__ __forceinline__ u32x2 gather4(const u32x4& r0, const u32x4& r1,
   return out;
 }
 
+// Maximum and sum over the lane pair (lane, lane ^ 32).  v_permlane32_swap
+// leaves the lower half's value in one register and the upper half's in the
+// other, for every lane: no trip through LDS (the shuffle is a ds_bpermute,
+// some 100 cycles of every key step's chain).
+__device__ __forceinline__ f32x2 wave_pair(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const uint32_t lo = r[0], hi = r[1];
+  return f32x2{__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi)};
+}
 __device__ __forceinline__ float wave_pair_max(float x) {
-  return fmaxf(x, __shfl_xor(x, 32));
+  const f32x2 p = wave_pair(x);
+  return fmaxf(p[0], p[1]);
 }
 __device__ __forceinline__ float wave_pair_sum(float x) {
-  return x + __shfl_xor(x, 32);
+  const f32x2 p = wave_pair(x);
+  return p[0] + p[1];
 }
 
 __device__ __forceinline__ int cdiv(int a, int b) { return (a + b - 1) / b; }

@@ -133,7 +133,7 @@ __device__ __forceinline__ void fwd_body(const FwdParams& P) {
   }
   auto issue = [&](int kt, uint8_t* base) {
     const int k0 = kt * C::BN;
-    const uint32_t rows = (uint32_t)max(min(C::BN, e.lk - k0), 0);
+    const uint32_t rows = (uint32_t)clamp_rows(e.lk - k0, C::BN);
     dk.issue(make_rsrc(kb + (int64_t)k0 * P.k.ss, rows * krb), base, wv);
     if constexpr (C::CR > 0) {
       // (a vanilla head's rank tile is a zero-size range: the DMA writes

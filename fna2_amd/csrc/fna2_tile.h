@@ -126,6 +126,7 @@ template <int ROWS, int C, int NWAVE>
 struct Dma {
   static constexpr int N = ROWS * C / 64;              // instructions per tile
   static constexpr int PER_WAVE = (N + NWAVE - 1) / NWAVE;
+  static constexpr bool EVEN = N % NWAVE == 0;         // (then no share needs a check)
   static_assert(ROWS * C % 64 == 0, "tile must be a whole number of 1 KB wave loads");
   static_assert(C % 4 == 0 && ROWS % 16 == 0, "tile shape");
 
@@ -199,7 +200,7 @@ struct Dma {
 #pragma unroll
     for (int j = 0; j < PER_WAVE; ++j) {
       const int i = wave + j * NWAVE;
-      if (i < N)
+      if (EVEN || i < N)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(lds + i * 1024), 16,
                                                  voff[j] + add, 0, 0, 0);
     }
@@ -210,7 +211,7 @@ struct Dma {
 #pragma unroll
     for (int j = 0; j < PER_WAVE; ++j) {
       const int i = wave + j * NWAVE;
-      if (i < N)
+      if (EVEN || i < N)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(lds + i * 1024), 16, voff[j], 0,
                                                  0, 0);
     }
