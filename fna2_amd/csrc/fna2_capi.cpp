@@ -976,7 +976,25 @@ struct DecSplit {
   int n = 1, keys = 32;
 };
 
-DecSplit dec_split(const fna2_decode_args& a) {
+// The library's split count.  The waves that run at once are at most four per
+// CU (what reads at the full rate) and what the ring's LDS leaves room for:
+// one round of them, since a second, partly filled one is waited for by
+// half the chip -- but four splits where the lengths differ (`ragged`), whose
+// longest sequences would be the whole time else -- and at least four steps a
+// split.  Measured, decode and merge, us, two rounds (the rule before) -> one:
+//   64 sequences x 4096, H16 R32      408 -> 401, ragged 312 -> 289
+//   64 x 4096, H32/8 R32 (3 a CU)     293 -> 282, ragged 232 -> 225
+//   16 x 2048, H16 R32                53.3 -> 51.3, ragged 41.2 -> 38.3
+//   40 x 3000, H8 d64 R32             53.2 -> 51.2, ragged 39.6 -> 35.8
+//   8 x 8192, H32/8, ragged           39.6 -> 34.5
+// Few units: a split's steps are a chain of load latencies that nothing else
+// hides, so down to one step each as long as the waves stay few (two per CU;
+// more and the merge and the waves' own start outweigh it).  Up to two steps
+// a second launch costs more than it saves.  (Four-step splits -> the rule's:
+// B2 H8/4 L496 d128 13.0 -> 9.0, B1 H16 L200 d64 10.0 -> 7.7, B1 H32/8 L4096
+// d128 10.7 -> 9.7; B1 H8 L64 6.4 whole, 8.3 in two; B4 H32/8 L2500: 20 splits
+// (640 waves) 12.2, 40 15.8.)
+DecSplit dec_split(const fna2_decode_args& a, bool ragged) {
   DecSplit s;
   const int64_t L = a.max_seqlen_k;
   if (L <= 0) return s;
@@ -986,16 +1004,9 @@ DecSplit dec_split(const fna2_decode_args& a) {
     const int rc = std::max(dec_rc(a), 0);
     const int per_cu = std::max(1, (160 * 1024) / (fna2::kDecodeStages *
                                                    fna2::decode_stage_bytes(a.head_dim, rc)));
-    const int64_t target = 2ll * kDecodeCUs * per_cu;  // two rounds of resident waves
-    n = std::min<int64_t>(cdiv64(target, units), cdiv64(L, 128));  // >= 4 steps a split
-    // Few units: a split's steps are a chain of load latencies that nothing
-    // else hides, so down to one step each as long as the waves stay few (two
-    // per CU; more and the merge and the waves' own start outweigh it).  Up
-    // to two steps a second launch costs more than it saves.  Measured (decode
-    // and merge, us, four-step splits -> the rule's): B2 H8/4 L496 d128 13.0 ->
-    // 9.0, B1 H16 L200 d64 10.0 -> 7.7, B1 H32/8 L4096 d128 10.7 -> 9.7; B1 H8
-    // L64 6.4 whole, 8.3 in two; B4 H32/8 L2500: 20 splits (640 waves) 12.2,
-    // 40 15.8.
+    n = (int64_t)kDecodeCUs * std::min(per_cu, 4) / units;
+    if (ragged) n = std::max<int64_t>(n, 4);
+    n = std::min<int64_t>(n, cdiv64(L, 128));
     if (L > 64) n = std::max<int64_t>(n, std::min<int64_t>(kDecodeFewWaves / units, cdiv64(L, 32)));
     n = std::max<int64_t>(std::min<int64_t>(n, 64), 1);
     if (L <= 64) n = 1;
@@ -1004,6 +1015,13 @@ DecSplit dec_split(const fna2_decode_args& a) {
   s.keys = (int)(cdiv64(cdiv64(L, n), 32) * 32);
   s.n = (int)cdiv64(L, s.keys);
   return s;
+}
+DecSplit dec_split(const fna2_decode_args& a) { return dec_split(a, a.seqlens_k != nullptr); }
+
+size_t dec_workspace(const fna2_decode_args& a, const DecSplit& s) {
+  if (s.n <= 1) return 0;
+  const size_t rows = (size_t)s.n * (size_t)a.batch * (size_t)a.heads;
+  return align_up(rows * (size_t)a.head_dim * 4u) + align_up(rows * 8u);
 }
 
 }  // namespace
@@ -1061,18 +1079,17 @@ int fna2_decode_num_splits(const fna2_decode_args* a) {
 
 size_t fna2_decode_workspace_bytes(const fna2_decode_args* a) {
   if (fna2_check_decode(a) != FNA2_OK) return 0;
-  const DecSplit s = dec_split(*a);
-  if (s.n <= 1) return 0;
-  const size_t rows = (size_t)s.n * (size_t)a->batch * (size_t)a->heads;
-  return align_up(rows * (size_t)a->head_dim * 4u) + align_up(rows * 8u);
+  return dec_workspace(*a, dec_split(*a));
 }
 
 int fna2_decode(const fna2_decode_args* a, void* stream_ptr) {
   FNA2_TRY(fna2_check_decode(a));
   if (a->batch == 0) return FNA2_OK;
   FNA2_TRY(check_device());
-  const DecSplit s = dec_split(*a);
-  const size_t need = fna2_decode_workspace_bytes(a);
+  // (a workspace sized without the lengths has the room of the even split)
+  DecSplit s = dec_split(*a);
+  if (dec_workspace(*a, s) > a->workspace_bytes) s = dec_split(*a, false);
+  const size_t need = dec_workspace(*a, s);
   if (need > 0 && (!a->workspace || a->workspace_bytes < need || !aligned(a->workspace, 16)))
     return FNA2_E_WORKSPACE;
   hipStream_t stream = (hipStream_t)stream_ptr;

@@ -26,9 +26,40 @@ def test_few_units_split_to_single_steps(L, n):
 
 
 def test_many_units_keep_long_splits():
-    assert _splits(64, 16, 16, 16, 128, 32, 4096) <= 3
+    assert _splits(64, 16, 16, 16, 128, 32, 4096) == 1
+    assert _splits(16, 16, 16, 16, 128, 32, 2048) == 4
     assert _splits(64, 16, 16, 16, 128, 32, 128) == 1
     assert _splits(8, 32, 8, 0, 128, 0, 1024) == 8
+
+
+@pytest.mark.gpu
+def test_workspace_sized_without_lengths(gpu):
+    """A ragged call may split more than the even one; with the even call's
+    workspace it splits as that does."""
+    from fna2_amd.decode import decode_args
+    g = torch.Generator().manual_seed(1)
+    mk = lambda *s: torch.randn(*s, generator=g).bfloat16().to(gpu)
+    B, H, L = 130, 8, 600
+    q, k, v = mk(B, H, 64), mk(B, H, L, 64), mk(B, H, L, 64)
+    seq = torch.tensor([(7 * i) % (L + 1) for i in range(B)], dtype=torch.int32, device=gpu)
+    lib = _capi.lib()
+    a, keep, out, _ = decode_args(q, k, v, cache_seqlens=seq)
+    big = lib.fna2_decode_workspace_bytes(ctypes.byref(a))
+    a.seqlens_k = None
+    small = lib.fna2_decode_workspace_bytes(ctypes.byref(a))
+    assert small < big
+    a.seqlens_k = keep[-1].data_ptr()
+    ws = torch.empty(big, dtype=torch.uint8, device=gpu)
+    a.workspace = ws.data_ptr()
+    outs = []
+    for n in (big, small):
+        a.workspace_bytes = n
+        st = lib.fna2_decode(ctypes.byref(a), torch.cuda.current_stream(gpu).cuda_stream)
+        assert st == 0
+        torch.cuda.synchronize()
+        outs.append(out.clone())
+    # (each split rounds P to bf16 against its own maximum)
+    assert (outs[0].float() - outs[1].float()).abs().max() <= 2 ** -7 * outs[0].float().abs().max()
 
 
 @pytest.mark.gpu
