@@ -108,6 +108,8 @@ struct KvCfg {
            ((m & kTileR) && RPL > 0 ? DmaR::PER_WAVE : 0) +
            ((m & kTileO) ? DmaD::PER_WAVE : 0) + ((m & kTileL) ? 1 : 0);
   }
+  // The producers' cursor moves in place (see there).
+  static constexpr bool INPLACE = !(D == 128 && RPL == 64);
   static constexpr int NBC = nb_of(CDMA);              // per consumer wave
   static constexpr int NBP = nb_of(kTileAll & ~CDMA);  // per producer wave
 };
@@ -567,10 +569,9 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
     // of the consumer's MFMAs: for k-half j (query rows 16j..16j+15), lane
     // (key l32, half hl) holds rows 16j + 8i + 4hl + e, i = 0..1, e = 0..3,
     // i.e. accumulator registers 8j..8j+7.
-    auto softmax = [&](const Cursor& c, uint8_t* pd, const f32x16 (&sacc_)[C::KPW],
+    // (qbase: the block's first query; k0t: the item's first key)
+    auto softmax = [&](int qbase, int k0t, uint8_t* pd, const f32x16 (&sacc_)[C::KPW],
                        const f32x16 (&dpacc_)[C::KPW], const f32x4_t (&lsr)[8]) {
-      const KvItem& x = c.it;
-      const int qbase = c.block() * C::BM;
 #pragma unroll
       for (int ks = 0; ks < C::KPW; ++ks) {
       const f32x16& sacc = sacc_[ks];
@@ -581,8 +582,8 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
       // query row qbase + r sees key k0t + krow iff r >= thr.  Blocks off
       // the diagonal (every block of a non-causal problem) skip the compare
       // and select, a fifth of the arithmetic per score.
-      const bool diag = p.causal && x.k0t + (kw * C::KPW + ks) * 32 + 31 > qbase;  // wave-uniform
-      const int thr = x.k0t + krow_of(ks) - qbase;
+      const bool diag = p.causal && k0t + (kw * C::KPW + ks) * 32 + 31 > qbase;  // wave-uniform
+      const int thr = k0t + krow_of(ks) - qbase;
       auto body = [&](auto masked) {
         u32x4 pk[2], dk[2], dr[2];
 #pragma unroll
@@ -672,31 +673,47 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
         sign_k();
         bhp = head_scale(pc);
       }
-      Cursor nx = pc;
-      advance(nx, no_zero);
+      Cursor nx;
       const bool act = block_active(pc);
+      const int qbase = pc.block() * C::BM, k0t = pc.it.k0t;
+      const bool seg_end = pc.qi + 1 >= pc.seg_blocks();
+      if constexpr (!C::INPLACE) {
+        nx = pc;
+        advance(nx, no_zero);
+      }
       f32x16 sacc[C::KPW], dpacc[C::KPW];
       f32x4_t lsr[8];
       __builtin_amdgcn_sched_barrier(0);
       if (act) scores(pc, cur, sacc, dpacc, lsr);
       __builtin_amdgcn_sched_barrier(0);
-      if (!nx.done && nx.qi == 0) {
+      // The cursor moves on in place, here, and only at a segment's end by
+      // more than its block count: a copy of it advanced every step cost the
+      // step some 30 scalar moves and selects (dK/dV, means of three runs: 32
+      // heads x 4096 d64 386 -> 375 us, d128 rank 32 367 -> 361, c2 111.7 ->
+      // 109.4).  At d = 128 and rank 64 the copy measured 3% faster and stays.
+      if (C::INPLACE ? seg_end : !nx.done && nx.qi == 0) {
         // The next (item, head)'s rows: after an (item, head) of two or more
         // blocks the consumers have DMA'd its K | Rk into LDS, and only V is
         // loaded here.
         // (One load site for each: branches around in-place loads of the
         // same registers made the compiler move them while in flight.)
         const bool from_lds = C::KR && pc.seg_blocks() >= 2;
-        load_k(nx.it, nx.it.kvh * p.group + nx.hi, from_lds);
-        load_v(nx.it);
-        kr_in = from_lds;
+        if constexpr (C::INPLACE) advance(pc, no_zero);
+        const Cursor& to = C::INPLACE ? pc : nx;
+        if (!to.done) {
+          load_k(to.it, to.it.kvh * p.group + to.hi, from_lds);
+          load_v(to.it);
+          kr_in = from_lds;
+        }
+      } else if constexpr (C::INPLACE) {
+        ++pc.qi;
       }
       __builtin_amdgcn_sched_barrier(0);
-      if (act) softmax(pc, pd, sacc, dpacc, lsr);
+      if (act) softmax(qbase, k0t, pd, sacc, dpacc, lsr);
       __builtin_amdgcn_sched_barrier(0);
       issue(nxt);
       __builtin_amdgcn_sched_barrier(0);
-      pc = nx;
+      if constexpr (!C::INPLACE) pc = nx;
     };
     // Block T uses stage T % 4 and P/dS buffer T % 2.  Steps 0 .. nblocks-1
     // produce; one more meets the consumers' last barrier.
