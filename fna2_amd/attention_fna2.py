@@ -724,15 +724,18 @@ class NaylisAttention(nn.Module):
     def _decode_rows(self, q, k, v, r_k, cache: StaticKVCache) -> Optional[torch.Tensor]:
         """The step's QK-RMSNorm, rotation and cache append in one launch:
         q's rows [B, H, 1, D], with the new rows in the cache; None where the
-        torch modules do it: with gradients or a tracer, in other dtypes, and
-        for a full cache or one without r_k (``append`` raises)."""
+        torch modules do it: with gradients, a tracer or module hooks, in other
+        dtypes, for a subclass of the cache (its ``append`` runs), and for a
+        full cache or one without r_k (``append`` raises)."""
         n = cache.length
-        if (torch.is_grad_enabled() or not _fna2_plain_eager(q) or n >= cache.capacity or
-                (cache.r_k is None) != (r_k is None)):
+        if (torch.is_grad_enabled() or not _fna2_plain_eager(q) or
+                type(cache) is not StaticKVCache or n >= cache.capacity or
+                (cache.r_k is None) != (r_k is None) or nn.modules.module._has_any_global_hook()):
             return None
         for m, cls in ((self.q_norm, RMSNorm), (self.k_norm, RMSNorm),
                        (self.rope, RotaryPositionalEmbedding)):
-            if m is not None and (type(m) is not cls or m._forward_hooks or m._forward_pre_hooks):
+            if m is not None and (type(m) is not cls or m._forward_hooks or
+                                  m._forward_pre_hooks or "forward" in vars(m)):
                 return None  # a replaced or hooked module is called as such
         cos = sin = None
         if self.rope is not None:

@@ -148,8 +148,8 @@ def flash_naylis_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.T
     ``[B, H]``).  ``num_splits`` 0 lets the library split the keys."""
     if q.is_cuda:  # the native launch path (None: a call it leaves to the code below)
         scale = q.shape[-1] ** -0.5 if softmax_scale is None else softmax_scale
-        done = _capi.native().decode(q, k_cache, v_cache, r_q, rk_cache, graph_scale, scale,
-                                     cache_seqlens, num_splits)
+        done = _capi.native().decode(q, k_cache, v_cache, r_q, rk_cache, graph_scale,
+                                     float(scale), cache_seqlens, int(num_splits))
         if done is not None:
             return done if return_lse else done[0]
     a, keep, out, lse = decode_args(q, k_cache, v_cache, r_q, rk_cache, graph_scale,

@@ -203,8 +203,9 @@ def _native_fwd(q, k, v, r_q, r_k, graph_scale, scale, causal, cu_q=None, cu_k=N
     per-kernel timing, errors to raise."""
     if _timer is not None or not q.is_cuda:
         return None
-    return _capi.native().attn_fwd(q, k, v, r_q, r_k, graph_scale, scale, bool(causal), cu_q, cu_k,
-                                   max_q, max_k, plan, bool(plan_filled), head_major)
+    return _capi.native().attn_fwd(q, k, v, r_q, r_k, graph_scale, float(scale), bool(causal),
+                                   cu_q, cu_k, int(max_q), int(max_k), plan, bool(plan_filled),
+                                   bool(head_major))
 
 
 def _native_bwd(dout, q, k, v, r_q, r_k, graph_scale, out, lse, scale, causal, cu_q=None,
@@ -215,8 +216,8 @@ def _native_bwd(dout, q, k, v, r_q, r_k, graph_scale, out, lse, scale, causal, c
     to = (None,) * 5 if grads_out is None else grads_out
     if to[0] is not None or to[1] is not None:
         return None
-    return _capi.native().attn_bwd(dout, q, k, v, r_q, r_k, graph_scale, out, lse, scale,
-                                   bool(causal), cu_q, cu_k, max_q, max_k, plan, *to[2:])
+    return _capi.native().attn_bwd(dout, q, k, v, r_q, r_k, graph_scale, out, lse, float(scale),
+                                   bool(causal), cu_q, cu_k, int(max_q), int(max_k), plan, *to[2:])
 
 
 def _workspace(fn, prob: _capi.Problem, dev) -> torch.Tensor:

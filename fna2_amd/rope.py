@@ -86,7 +86,8 @@ def rope_varlen_raw(q: torch.Tensor, k: torch.Tensor, cu_seqlens: torch.Tensor,
     """(Optionally RMS-normalise, then) rotate q ``[T, H, D]`` and k
     ``[T, H_KV, D]`` (no autograd); new tensors."""
     if q.is_cuda:  # the native launch path (None: a call it leaves to the code below)
-        done = _capi.native().rope_fwd(q, k, cu_seqlens, inv_freq, sign, norm_q, norm_k, eps)
+        done = _capi.native().rope_fwd(q, k, cu_seqlens, inv_freq, int(sign), norm_q, norm_k,
+                                       float(eps))
         if done is not None:
             return done
     q, k = _usable(q), _usable(k)
@@ -110,8 +111,8 @@ def rope_varlen_bwd(dq_out, dk_out, q, k, cu_seqlens, inv_freq, sign=1, norm_q=N
     tensors of q's and k's shapes to write into (any row strides, unit last
     stride), else new ones."""
     if q.is_cuda:
-        done = _capi.native().rope_bwd(dq_out, dk_out, q, k, cu_seqlens, inv_freq, sign, norm_q,
-                                       norm_k, eps, dq, dk)
+        done = _capi.native().rope_bwd(dq_out, dk_out, q, k, cu_seqlens, inv_freq, int(sign),
+                                       norm_q, norm_k, float(eps), dq, dk)
         if done is not None:
             return done
     q, k = _usable(q), _usable(k)

@@ -116,8 +116,8 @@ def test_module_step_against_torch_modules(gpu, bias, kw):
     x = torch.randn(3, 1, 512, device=gpu).bfloat16()
     kv = kw.get("n_kv_heads", 8)
 
-    def step(fused):
-        c = A.StaticKVCache.empty(3, kv, 12, 64, 8 if bias else 0, 16, device=gpu)
+    def step(fused, cls=A.StaticKVCache):
+        c = cls.empty(3, kv, 12, 64, 8 if bias else 0, 16, device=gpu)
         g = torch.Generator(device=gpu).manual_seed(1)
         rows = [torch.randn(3, h, 10, f, device=gpu, generator=g).bfloat16()
                 for h, f in ((kv, 64), (kv, 64)) + (((8, 16),) if bias else ())]
@@ -141,6 +141,21 @@ def test_module_step_against_torch_modules(gpu, bias, kw):
         step(True)
         h.remove()
         assert calls
+        h = torch.nn.modules.module.register_module_forward_pre_hook(
+            lambda mod, a: calls.append(mod))
+        step(True)
+        h.remove()
+        assert m.q_norm in calls
+    # a cache of another class appends by its own method
+
+    class Cache(A.StaticKVCache):
+        n = 0
+
+        def append(self, *rows):
+            Cache.n += 1
+            super().append(*rows)
+    step(True, Cache)
+    assert Cache.n == 2
     full = A.StaticKVCache.empty(3, kv, 4, 64, 8 if bias else 0, 16, device=gpu)
     full.length = 4
     with pytest.raises(ValueError, match="full"), torch.no_grad():

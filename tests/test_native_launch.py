@@ -114,3 +114,19 @@ def test_calls_left_to_the_python_launcher(gpu):
         F._fna2_forward(q, k.half(), v, rq, rk, gs, s, True)
     with pytest.raises(AssertionError, match="FNA2_E_SCALE"):
         F._fna2_forward(q, k, v, rq, rk, gs, float("nan"), True)
+
+
+@pytest.mark.gpu
+def test_numbers_of_other_types(gpu):
+    """The numbers that the Python launchers convert: any real or integral
+    object, also a float that holds a count."""
+    from fna2_amd.decode import flash_naylis_decode
+    q, k, v, rq, rk, gs, dout = [t.to(gpu) for t in Hp.make_dense(1, 4, 64, 64, 4, 4, 16)]
+    ref = flash_naylis_decode(q[:, :, 0], k, v, softmax_scale=0.125, num_splits=2)
+    got = flash_naylis_decode(q[:, :, 0], k, v, softmax_scale=torch.tensor(0.125), num_splits=2.0)
+    assert torch.equal(got, ref)
+    x = [t[0].transpose(0, 1).contiguous() for t in (q, k, v, rq, rk)]
+    cu = torch.tensor([0, 40, 64], dtype=torch.int32, device=gpu)
+    ref = F._fna2_forward_varlen(*x, gs, cu, cu, 40, 40, 0.125, True)
+    got = F._fna2_forward_varlen(*x, gs, cu, cu, 40.0, torch.tensor(40), torch.tensor(0.125), 1)
+    assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
