@@ -87,3 +87,20 @@ def test_merge_of_n_splits(gpu, n, D, R):
     assert (l - l1)[fin].abs().max() < 1e-5
     assert not o[2].any()
     assert torch.equal(run(n)[0], o)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [1, 2, 7])
+@pytest.mark.parametrize("D", [64, 128])
+def test_error_is_the_outputs_rounding(gpu, D, splits):
+    """The probabilities enter their product with 16 bits of significand, so
+    the error is the bf16 output's rounding, at most 2^-9 of each value (and
+    2^-16 for what P's second part and the fp32 sums leave)."""
+    from fna2_amd.decode import flash_naylis_decode
+    g = torch.Generator().manual_seed(D + splits)
+    q, k, v = (torch.randn(*s, generator=g).bfloat16() for s in
+               ((3, 8, D), (3, 4, 1500, D), (3, 4, 1500, D)))
+    s = q.double().view(3, 4, 2, D) @ k.double().transpose(2, 3) * D ** -0.5
+    ref = (torch.softmax(s, -1) @ v.double()).view(3, 8, D)
+    got = flash_naylis_decode(q.to(gpu), k.to(gpu), v.to(gpu), num_splits=splits).cpu().double()
+    assert (got - ref).norm() <= (2 ** -9 + 2 ** -16) * ref.norm()
