@@ -979,14 +979,18 @@ struct DecSplit {
 // The library's split count.  The waves that run at once are at most four per
 // CU (what reads at the full rate) and what the ring's LDS leaves room for:
 // one round of them, since a second, partly filled one is waited for by
-// half the chip -- but four splits where the lengths differ (`ragged`), whose
-// longest sequences would be the whole time else -- and at least four steps a
-// split.  Measured, decode and merge, us, two rounds (the rule before) -> one:
-//   64 sequences x 4096, H16 R32      408 -> 401, ragged 312 -> 289
-//   64 x 4096, H32/8 R32 (3 a CU)     293 -> 282, ragged 232 -> 225
-//   16 x 2048, H16 R32                53.3 -> 51.3, ragged 41.2 -> 38.3
-//   40 x 3000, H8 d64 R32             53.2 -> 51.2, ragged 39.6 -> 35.8
-//   8 x 8192, H32/8, ragged           39.6 -> 34.5
+// half the chip -- and at least four steps a split.  Where the lengths differ
+// (`ragged`) the longest sequences would be the whole time: four splits at
+// least, eight where a round holds fewer than four (several rounds then, whose
+// later waves level the lengths).  Measured, decode and merge, us, two rounds
+// (the rule before) -> this one, ragged as the mean of three draws:
+//   64 sequences x 4096, H16 R32      403 -> 397, ragged 264 -> 243 (4: 244)
+//   64 x 4096, H32/8 R32 (3 a CU)     285 -> 278, ragged 211 -> 191 (4: 182)
+//   16 x 2048, H16 R32                54.9 -> 55.2, ragged 41.4 -> 36.6
+//   24 x 5000, H16 R32                211 -> 192, ragged 133 -> 124 (4: 127)
+//   15 x 5065, H32                    216 -> 212, ragged 146 -> 147 (4: 156)
+//   48 x 3000, H16 d64                108 -> 102, ragged 69 -> 68 (4: 71)
+//   20 x 6000, H32/8                  100 -> 91, ragged 57 -> 54
 // Few units: a split's steps are a chain of load latencies that nothing else
 // hides, so down to one step each as long as the waves stay few (two per CU;
 // more and the merge and the waves' own start outweigh it).  Up to two steps
@@ -1005,7 +1009,7 @@ DecSplit dec_split(const fna2_decode_args& a, bool ragged) {
     const int per_cu = std::max(1, (160 * 1024) / (fna2::kDecodeStages *
                                                    fna2::decode_stage_bytes(a.head_dim, rc)));
     n = (int64_t)kDecodeCUs * std::min(per_cu, 4) / units;
-    if (ragged) n = std::max<int64_t>(n, 4);
+    if (ragged) n = std::max<int64_t>(n, n < 4 ? 8 : 4);
     n = std::min<int64_t>(n, cdiv64(L, 128));
     if (L > 64) n = std::max<int64_t>(n, std::min<int64_t>(kDecodeFewWaves / units, cdiv64(L, 32)));
     n = std::max<int64_t>(std::min<int64_t>(n, 64), 1);
