@@ -725,10 +725,12 @@ class NaylisAttention(nn.Module):
         """The step's QK-RMSNorm, rotation and cache append in one launch:
         q's rows [B, H, 1, D], with the new rows in the cache; None where the
         torch modules do it: with gradients, a tracer or module hooks, in other
-        dtypes, for a subclass of the cache (its ``append`` runs), and for a
+        dtypes, under autocast (which forms the norm and so the rotary table
+        in fp32), for a subclass of the cache (its ``append`` runs), and for a
         full cache or one without r_k (``append`` raises)."""
         n = cache.length
         if (torch.is_grad_enabled() or not _fna2_plain_eager(q) or
+                torch.is_autocast_enabled(q.device.type) or
                 type(cache) is not StaticKVCache or n >= cache.capacity or
                 (cache.r_k is None) != (r_k is None) or nn.modules.module._has_any_global_hook()):
             return None

@@ -160,3 +160,43 @@ def test_module_step_against_torch_modules(gpu, bias, kw):
     full.length = 4
     with pytest.raises(ValueError, match="full"), torch.no_grad():
         m(x, past_kv=full, use_kv_cache=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kw", [dict(), dict(use_qk_norm=False)], ids=str)
+def test_step_under_autocast(gpu, kw):
+    """Under autocast the norm's square and root run in fp32, and with them
+    the rotary table: the step is the torch modules', and the row it appends
+    is rotated by exact angles, as the prompt's rows are."""
+    from fna2_amd import attention_fna2 as A
+    torch.manual_seed(0)
+    m = A.NaylisAttention(256, 4, rel_rank=16, max_seq_len=512, decode_graph_bias=True,
+                          **kw).to(gpu).bfloat16().eval()
+    x = torch.randn(2, 1, 256, device=gpu).bfloat16()
+    n = 257
+
+    def step(fused):
+        g = torch.Generator(device=gpu).manual_seed(1)
+        c = A.StaticKVCache.empty(2, 4, n + 1, 64, 4, 16, device=gpu)
+        c.append(*(torch.randn(2, 4, n, f, device=gpu, generator=g).bfloat16() for f in (64, 64, 16)))
+        if not fused:
+            m._decode_rows = lambda *a: None
+        try:
+            with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+                y, _ = m(x, past_kv=c, use_kv_cache=True)
+        finally:
+            m.__dict__.pop("_decode_rows", None)
+        return y, c.k[:, :, n]
+    if kw:  # without the norm nothing is promoted: the bf16 table on both sides
+        for a, b in zip(step(True), step(False)):
+            assert (a.double() - b.double()).norm() <= 0.015 * b.double().norm()
+        return
+    (y, k), (y0, k0) = step(True), step(False)
+    assert torch.equal(k, k0) and torch.equal(y, y0)
+    with torch.no_grad():
+        kk = m._project(x)[1].double()
+        kk = kk * torch.rsqrt(kk.square().mean(-1, keepdim=True) + 1e-6) * m.k_norm.weight.double()
+        ang = n * m.rope.inv_freq.double()
+        c, s = ang.cos().repeat(2), ang.sin().repeat(2)
+        h = torch.cat((-kk[..., 32:], kk[..., :32]), -1)
+    assert (k.double() - (kk * c + h * s)[:, :, 0]).norm() <= 2 ** -7 * k.double().norm()
