@@ -228,11 +228,14 @@ __device__ __forceinline__ void decode_body(const DecodeParams& P) {
     const float m_use = (m_new == kNegInf) ? 0.f : m_new;
     const float nm = -m_use * P.c2;
     float ls = 0.f;
-    // P as bf16 plus the bf16 of what that rounding left, so that the result
+    // P as bf16 plus the bf16 of what that cut off, so that the result
     // does not depend on the split count: with P in bf16 alone a split's own
     // maximum (P = 1) is exact, and fewer splits meant fewer such keys
     // (relative error against fp64, 4096 keys: 0.00200
     // in 8 splits, 0.00215 in one; now 0.00166 in any, the output's rounding).
+    // The first part is cut, not rounded, and the second has its last bit
+    // set: it is never negative or zero, either of which would turn an
+    // infinite V into NaN.  (At most 2^-14 of P.)
     // The kernel waits for memory, not for the second product: 64 x 4096
     // 401.1 -> 401.6 us, GQA 280.8 -> 279.2, 4 x 2500 11.9 -> 12.3, 8 x 8192
     // ragged GQA 52.1 -> 55.5.
@@ -246,10 +249,10 @@ __device__ __forceinline__ void decode_body(const DecodeParams& P) {
         const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[v0], P.c2, nm));
         const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[v0 + 1], P.c2, nm));
         ls += p0 + p1;
-        const uint32_t w = pack_bf16(p0, p1);
-        pk[i] = w;
-        ek[i] = pack_bf16(p0 - __builtin_bit_cast(float, w << 16),
-                          p1 - __builtin_bit_cast(float, w & 0xffff0000u));
+        const uint32_t u0 = __builtin_bit_cast(uint32_t, p0), u1 = __builtin_bit_cast(uint32_t, p1);
+        pk[i] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // their upper halves
+        ek[i] = pack_bf16(p0 - __builtin_bit_cast(float, u0 & 0xffff0000u),
+                          p1 - __builtin_bit_cast(float, u1 & 0xffff0000u)) | 0x00010001u;
       }
       pb[half] = as_bf16x8(pk);
       pe[half] = as_bf16x8(ek);

@@ -104,3 +104,39 @@ def test_error_is_the_outputs_rounding(gpu, D, splits):
     ref = (torch.softmax(s, -1) @ v.double()).view(3, 8, D)
     got = flash_naylis_decode(q.to(gpu), k.to(gpu), v.to(gpu), num_splits=splits).cpu().double()
     assert (got - ref).norm() <= (2 ** -9 + 2 ** -16) * ref.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("D,R", [(64, 0), (128, 32)])
+def test_infinite_values(gpu, D, R, splits):
+    """An infinite V gives an infinite output where its key has weight, as
+    torch does, also at a split's maximum (P = 1, no second part) and where P
+    rounds up to bf16; NaN stays in its feature."""
+    from fna2_amd.decode import flash_naylis_decode
+    g = torch.Generator().manual_seed(D + splits)
+    B, H, HKV, L = 2, 4, 2, 200
+    q, k, v = (torch.randn(*s, generator=g).bfloat16() for s in
+               ((B, H, D), (B, HKV, L, D), (B, HKV, L, D)))
+    bias = ()
+    if R:
+        bias = (torch.randn(B, H, R, generator=g).bfloat16() * R ** -0.5,
+                torch.randn(B, H, L, R, generator=g).bfloat16(), torch.ones(H))
+    s = (q.double().view(B, HKV, 2, D) @ k.double().transpose(2, 3)).view(B, H, L) * D ** -0.5
+    if R:
+        s += (bias[1].double() @ bias[0].double()[..., None])[..., 0]
+    top = s[0, 0].argmax().item()
+    inf = float("inf")
+    v[0, 0, top, 3] = inf
+    for j in range(8):  # eight keys' weights: rounded up, rounded down
+        v[0, 1, 17 + 23 * j, 5 + j] = inf if j % 2 else -inf
+    v[1, 0, 199, D - 1] = -inf
+    v[1, 1, 40, 8], v[1, 1, 41, 8] = inf, -inf
+    v[1, 1, 0, 9] = float("nan")
+    ref = (torch.softmax(s, -1).view(B, HKV, 2, L) @ v.double()).view(B, H, D)
+    got = flash_naylis_decode(*(t.to(gpu) for t in (q, k, v, *bias)), num_splits=splits).cpu()
+    fin = torch.isfinite(ref)
+    assert (~fin).sum() == 2 * (1 + 8 + 1 + 1 + 1)
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(got.double()[~fin & ~torch.isnan(ref)], ref[~fin & ~torch.isnan(ref)])
+    assert (got.double() - ref)[fin].norm() <= 2 ** -8 * ref[fin].norm()
