@@ -739,6 +739,9 @@ class NaylisAttention(nn.Module):
             if m is not None and (type(m) is not cls or m._forward_hooks or
                                   m._forward_pre_hooks or "forward" in vars(m)):
                 return None  # a replaced or hooked module is called as such
+        if not q.is_cuda or any(t.dtype != torch.bfloat16 for t in (
+                q, *(m.weight for m in (self.q_norm, self.k_norm) if m is not None))):
+            return None  # (the modules' table is then of another dtype: see _table)
         cos = sin = None
         if self.rope is not None:
             cos, sin = self.rope._table(n + 1, q.device, q.dtype)

@@ -200,3 +200,19 @@ def test_step_under_autocast(gpu, kw):
         c, s = ang.cos().repeat(2), ang.sin().repeat(2)
         h = torch.cat((-kk[..., 32:], kk[..., :32]), -1)
     assert (k.double() - (kk * c + h * s)[:, :, 0]).norm() <= 2 ** -7 * k.double().norm()
+
+
+def test_rotary_table_is_left_alone():
+    """A step that the torch modules take (here fp32 norm weights over bf16
+    projections, CPU tensors) does not touch the rotary table: the table
+    holds one dtype, and two callers of two dtypes would rebuild it each step."""
+    from fna2_amd import attention_fna2 as A
+    m = A.NaylisAttention(128, 2, rel_rank=16, max_seq_len=64).bfloat16().eval()
+    m.q_norm.float()
+    m.k_norm.float()
+    c = A.StaticKVCache.empty(1, 2, 8, 64, 0, 16, device="cpu")
+    c.append(torch.zeros(1, 2, 4, 64).bfloat16(), torch.zeros(1, 2, 4, 64).bfloat16())
+    with torch.no_grad():
+        q, k, v, _, _ = m._project(torch.randn(1, 1, 128).bfloat16())
+        assert m._decode_rows(q, k, v, None, c) is None
+    assert m.rope._cache_key is None and c.length == 4
