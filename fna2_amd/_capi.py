@@ -252,6 +252,10 @@ def lib() -> ctypes.CDLL:
 _native = None
 
 
+def _addresses(handle: ctypes.CDLL) -> dict:
+    return {n: ctypes.cast(getattr(handle, n), ctypes.c_void_p).value for n in SIGNATURES}
+
+
 def native():
     """The torch binding (``csrc/fna2_torch.cpp``), bound to ``lib()``'s
     functions.  Raises if it has not been built."""
@@ -264,7 +268,7 @@ def native():
         except ImportError as e:
             raise RuntimeError("fna2_amd/_torch_binding.so does not load; build it with "
                                f"`python -m fna2_amd.build` ({e})") from e
-        mod.bind({n: ctypes.cast(getattr(handle, n), ctypes.c_void_p).value for n in SIGNATURES})
+        mod.bind(_addresses(handle), FNA2Error)
         _native = mod
     return _native
 

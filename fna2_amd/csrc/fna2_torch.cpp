@@ -13,7 +13,9 @@
 // shapes and dtypes, on one device, laid out as the kernels read them.  For
 // anything else, and for a call the C ABI refuses (nothing is launched
 // then), it returns None, and the caller's Python launcher makes the copies
-// or raises the error, as without this file.
+// or raises the error, as without this file.  A launch that fails raises
+// here: other kernels of the call may be queued by then, so it is not
+// repeated.
 //
 // The library's functions come as addresses (bind), so that the binding
 // always calls the library that _capi.py loaded.
@@ -49,7 +51,20 @@ struct Lib {
 };
 Lib L{};
 
-void bind(const std::map<std::string, uintptr_t>& f) {
+PyObject* launch_error = nullptr;  // the exception class (never freed)
+
+// Whether a call was launched; false where the C ABI refused it.
+bool launched(int status, const char* what) {
+  if (status == FNA2_E_LAUNCH) {
+    const py::gil_scoped_acquire gil;
+    PyErr_Format(launch_error, "%s: FNA2_E_LAUNCH: kernel launch failed", what);
+    throw py::error_already_set();
+  }
+  return status == FNA2_OK;
+}
+
+void bind(const std::map<std::string, uintptr_t>& f, py::object error) {
+  launch_error = error.release().ptr();
 #define FNA2_BIND(n) L.n = reinterpret_cast<decltype(L.n)>(f.at("fna2_" #n))
   FNA2_BIND(fwd);
   FNA2_BIND(bwd);
@@ -215,7 +230,7 @@ std::optional<std::tuple<Tensor, Tensor>> attn_fwd(
     a.plan_bytes = (size_t)plan.numel();
     a.plan_filled = plan_filled;
   }
-  if (L.fwd(&a, stream_of(q.device())) != FNA2_OK) return std::nullopt;
+  if (!launched(L.fwd(&a, stream_of(q.device())), "fna2_fwd")) return std::nullopt;
   return std::make_tuple(out, lse);
 }
 
@@ -286,7 +301,7 @@ std::optional<Grads> attn_bwd(const Tensor& dout, const Tensor& q, const Tensor&
     a.plan = plan.data_ptr();
     a.plan_bytes = (size_t)plan.numel();
   }
-  if (L.bwd(&a, stream_of(dev)) != FNA2_OK) return std::nullopt;
+  if (!launched(L.bwd(&a, stream_of(dev)), "fna2_bwd")) return std::nullopt;
   auto some = [](const Tensor& t) { return t.defined() ? OptTensor(t) : std::nullopt; };
   return Grads(dq, dk, dv, some(drq), some(drk), some(dgs));
 }
@@ -370,7 +385,7 @@ std::optional<std::tuple<Tensor, Tensor>> decode(const Tensor& q_, const Tensor&
     a.workspace = ws.data_ptr();
     a.workspace_bytes = need;
   }
-  if (L.decode(&a, stream_of(dev)) != FNA2_OK) return std::nullopt;
+  if (!launched(L.decode(&a, stream_of(dev)), "fna2_decode")) return std::nullopt;
   return std::make_tuple(out, lse);
 }
 
@@ -436,7 +451,7 @@ OptTensor decode_rows(const Tensor& q, const Tensor& k, const Tensor& v, const O
   a.v_out = row_view(v_out);
   a.eps_q = (float)eps_q;
   a.eps_k = (float)eps_k;
-  if (L.decode_rows(&a, stream_of(dev)) != FNA2_OK) return std::nullopt;
+  if (!launched(L.decode_rows(&a, stream_of(dev)), "fna2_decode_rows")) return std::nullopt;
   for (const Tensor* t : written)
     if (t && !t->is_inference()) t->unsafeGetTensorImpl()->bump_version();
   return out;
@@ -494,7 +509,7 @@ std::optional<std::tuple<Tensor, Tensor>> rope_fwd(const Tensor& q, const Tensor
   const Tensor ko = at::empty_like(k, at::MemoryFormat::Contiguous);
   a.q_out = view(qo, true);
   a.k_out = view(ko, true);
-  if (L.rope_varlen(&a, stream_of(q.device())) != FNA2_OK) return std::nullopt;
+  if (!launched(L.rope_varlen(&a, stream_of(q.device())), "fna2_rope_varlen")) return std::nullopt;
   return std::make_tuple(qo, ko);
 }
 
@@ -532,7 +547,7 @@ std::optional<std::tuple<Tensor, Tensor, OptTensor, OptTensor>> rope_bwd(
     b.workspace = ws.data_ptr();
     b.workspace_bytes = need;
   }
-  if (L.rope_bwd(&b, stream_of(dev)) != FNA2_OK) return std::nullopt;
+  if (!launched(L.rope_bwd(&b, stream_of(dev)), "fna2_rope_bwd")) return std::nullopt;
   return std::make_tuple(dq, dk, dn[0], dn[1]);
 }
 

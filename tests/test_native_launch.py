@@ -130,3 +130,47 @@ def test_numbers_of_other_types(gpu):
     ref = F._fna2_forward_varlen(*x, gs, cu, cu, 40, 40, 0.125, True)
     got = F._fna2_forward_varlen(*x, gs, cu, cu, 40.0, torch.tensor(40), torch.tensor(0.125), 1)
     assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
+
+
+@pytest.mark.gpu
+def test_failed_launch_is_raised_not_repeated(gpu, native):
+    """FNA2_E_LAUNCH may come after other kernels of the call were queued:
+    it is raised, and no Python launcher or torch module runs the call again."""
+    import ctypes
+
+    from fna2_amd import _capi, attention_fna2 as A, decode as De, rope as Ro
+    q, k, v, rq, rk, gs, dout = [t.to(gpu) for t in Hp.make_dense(1, 4, 64, 64, 4, 4, 16)]
+    out, lse = F._fna2_forward(q, k, v, rq, rk, gs, 0.125, True)
+    x = q[0].transpose(0, 1).contiguous()
+    cu = torch.tensor([0, 64], dtype=torch.int32, device=gpu)
+    inv = torch.ones(32, device=gpu)
+    m = A.NaylisAttention(256, 4, rel_rank=16, max_seq_len=64).to(gpu).bfloat16().eval()
+    cache = A.StaticKVCache.empty(1, 4, 8, 64, device=gpu)
+    cache.length = 3
+    row = torch.zeros(1, 1, 256, device=gpu).bfloat16()
+    step = torch.no_grad()(lambda: m(row, past_kv=cache, use_kv_cache=True))
+    calls = [("fna2_fwd", lambda: F._fna2_forward(q, k, v, rq, rk, gs, 0.125, True)),
+             ("fna2_bwd", lambda: F._fna2_backward(dout, q, k, v, rq, rk, gs, out, lse, 0.125, True)),
+             ("fna2_decode", lambda: De.flash_naylis_decode(q[:, :, 0], k, v)),
+             ("fna2_decode_rows", step),
+             ("fna2_rope_varlen", lambda: Ro.rope_varlen_raw(x, x, cu, inv)),
+             ("fna2_rope_bwd", lambda: Ro.rope_varlen_bwd(x, x, x, x, cu, inv))]
+    n = [0]
+
+    @ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p)
+    def fails(args, stream):
+        n[0] += 1
+        return -10
+    good = _capi._addresses(_capi.lib())
+    for name, call in calls:
+        print(name, flush=True)
+        native.bind({**good, name: ctypes.cast(fails, ctypes.c_void_p).value}, _capi.FNA2Error)
+        try:
+            n[0] = 0
+            with pytest.raises(_capi.FNA2Error, match=f"{name}: FNA2_E_LAUNCH"):
+                call()
+            assert n[0] == 1
+        finally:
+            native.bind(good, _capi.FNA2Error)
+        call()
+    assert cache.length == 4
