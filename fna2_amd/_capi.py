@@ -12,6 +12,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(os.environ.get("FNA2_LIB", Path(__file__).resolve().parent / "libfna2_hip.so"))
@@ -271,6 +272,27 @@ def native():
         mod.bind(_addresses(handle), FNA2Error)
         _native = mod
     return _native
+
+
+_native_missing = False
+
+
+def native_or_none():
+    """``native()``; None, after one warning, where the library loads but the
+    binding does not (not built, or built against another torch): the Python
+    launchers then make every call, slower by their host time."""
+    global _native_missing
+    if _native is not None:
+        return _native
+    if _native_missing:
+        return None
+    lib()
+    try:
+        return native()
+    except RuntimeError as e:
+        _native_missing = True
+        warnings.warn(f"{e}; calls go through the Python launchers", RuntimeWarning, stacklevel=3)
+        return None
 
 
 def available() -> bool:

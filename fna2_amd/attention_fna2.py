@@ -42,7 +42,6 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _capi
-from ._capi import native as _native
 from .flash_naylis_attn import BLOCK_R, flash_naylis_attn, rank_supported
 from .flash_naylis_attn import FlashNaylisAttnFunc as _FNA2Func
 from .flash_naylis_attn import _plain_eager as _fna2_plain_eager
@@ -739,7 +738,8 @@ class NaylisAttention(nn.Module):
             if m is not None and (type(m) is not cls or m._forward_hooks or
                                   m._forward_pre_hooks or "forward" in vars(m)):
                 return None  # a replaced or hooked module is called as such
-        if not q.is_cuda or any(t.dtype != torch.bfloat16 for t in (
+        nat = _capi.native_or_none() if q.is_cuda else None
+        if nat is None or any(t.dtype != torch.bfloat16 for t in (
                 q, *(m.weight for m in (self.q_norm, self.k_norm) if m is not None))):
             return None  # (the modules' table is then of another dtype: see _table)
         cos = sin = None
@@ -747,7 +747,7 @@ class NaylisAttention(nn.Module):
             cos, sin = self.rope._table(n + 1, q.device, q.dtype)
             cos, sin = cos[n], sin[n]
         norm = self.use_qk_norm
-        out = _native().decode_rows(
+        out = nat.decode_rows(
             q, k, v, r_k, cache.k[:, :, n:n + 1], cache.v[:, :, n:n + 1],
             None if r_k is None else cache.r_k[:, :, n:n + 1],
             self.q_norm.weight if norm else None, self.q_norm.eps if norm else 0.0,

@@ -146,10 +146,11 @@ def flash_naylis_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.T
     graph_scale ``[H_G]``, cache_seqlens ``[B]`` (rows in use, <= L; None:
     all L).  bf16.  Returns out ``[B, H, D]`` bf16 (and the fp32 LSE
     ``[B, H]``).  ``num_splits`` 0 lets the library split the keys."""
-    if q.is_cuda:  # the native launch path (None: a call it leaves to the code below)
+    nat = _capi.native_or_none() if q.is_cuda else None
+    if nat is not None:  # the native launch path (None: a call it leaves to the code below)
         scale = q.shape[-1] ** -0.5 if softmax_scale is None else softmax_scale
-        done = _capi.native().decode(q, k_cache, v_cache, r_q, rk_cache, graph_scale,
-                                     float(scale), cache_seqlens, int(num_splits))
+        done = nat.decode(q, k_cache, v_cache, r_q, rk_cache, graph_scale, float(scale),
+                          cache_seqlens, int(num_splits))
         if done is not None:
             return done if return_lse else done[0]
     a, keep, out, lse = decode_args(q, k_cache, v_cache, r_q, rk_cache, graph_scale,

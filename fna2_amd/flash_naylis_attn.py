@@ -201,23 +201,22 @@ def _native_fwd(q, k, v, r_q, r_k, graph_scale, scale, causal, cu_q=None, cu_k=N
     """(out, lse) by the native launch path, or None for the calls it leaves
     to the Python launcher: layouts and dtypes to convert, empty tensors,
     per-kernel timing, errors to raise."""
-    if _timer is not None or not q.is_cuda:
+    nat = _capi.native_or_none() if _timer is None and q.is_cuda else None
+    if nat is None:
         return None
-    return _capi.native().attn_fwd(q, k, v, r_q, r_k, graph_scale, float(scale), bool(causal),
-                                   cu_q, cu_k, int(max_q), int(max_k), plan, bool(plan_filled),
-                                   bool(head_major))
+    return nat.attn_fwd(q, k, v, r_q, r_k, graph_scale, float(scale), bool(causal), cu_q, cu_k,
+                        int(max_q), int(max_k), plan, bool(plan_filled), bool(head_major))
 
 
 def _native_bwd(dout, q, k, v, r_q, r_k, graph_scale, out, lse, scale, causal, cu_q=None,
                 cu_k=None, max_q=0, max_k=0, plan=None, grads_out=None):
     """The backward's gradients by the native launch path, or None (as above)."""
-    if _timer is not None or not q.is_cuda:
-        return None
+    nat = _capi.native_or_none() if _timer is None and q.is_cuda else None
     to = (None,) * 5 if grads_out is None else grads_out
-    if to[0] is not None or to[1] is not None:
+    if nat is None or to[0] is not None or to[1] is not None:
         return None
-    return _capi.native().attn_bwd(dout, q, k, v, r_q, r_k, graph_scale, out, lse, float(scale),
-                                   bool(causal), cu_q, cu_k, int(max_q), int(max_k), plan, *to[2:])
+    return nat.attn_bwd(dout, q, k, v, r_q, r_k, graph_scale, out, lse, float(scale),
+                        bool(causal), cu_q, cu_k, int(max_q), int(max_k), plan, *to[2:])
 
 
 def _workspace(fn, prob: _capi.Problem, dev) -> torch.Tensor:

@@ -85,9 +85,9 @@ def rope_varlen_raw(q: torch.Tensor, k: torch.Tensor, cu_seqlens: torch.Tensor,
                     eps: float = 1e-6) -> Tuple[torch.Tensor, torch.Tensor]:
     """(Optionally RMS-normalise, then) rotate q ``[T, H, D]`` and k
     ``[T, H_KV, D]`` (no autograd); new tensors."""
-    if q.is_cuda:  # the native launch path (None: a call it leaves to the code below)
-        done = _capi.native().rope_fwd(q, k, cu_seqlens, inv_freq, int(sign), norm_q, norm_k,
-                                       float(eps))
+    nat = _capi.native_or_none() if q.is_cuda else None
+    if nat is not None:  # the native launch path (None: a call it leaves to the code below)
+        done = nat.rope_fwd(q, k, cu_seqlens, inv_freq, int(sign), norm_q, norm_k, float(eps))
         if done is not None:
             return done
     q, k = _usable(q), _usable(k)
@@ -110,9 +110,10 @@ def rope_varlen_bwd(dq_out, dk_out, q, k, cu_seqlens, inv_freq, sign=1, norm_q=N
     gradients of its outputs (q, k: its inputs, needed with a norm).  dq, dk:
     tensors of q's and k's shapes to write into (any row strides, unit last
     stride), else new ones."""
-    if q.is_cuda:
-        done = _capi.native().rope_bwd(dq_out, dk_out, q, k, cu_seqlens, inv_freq, int(sign),
-                                       norm_q, norm_k, float(eps), dq, dk)
+    nat = _capi.native_or_none() if q.is_cuda else None
+    if nat is not None:
+        done = nat.rope_bwd(dq_out, dk_out, q, k, cu_seqlens, inv_freq, int(sign), norm_q, norm_k,
+                            float(eps), dq, dk)
         if done is not None:
             return done
     q, k = _usable(q), _usable(k)

@@ -26,6 +26,54 @@ def test_cpu_tensors_are_left_to_the_python_launchers(native):
         F._fna2_forward(t, t, t, None, None, None, 0.1, True)
 
 
+def test_without_the_binding_the_python_launchers_run(monkeypatch):
+    """A tree with the library and no (or another torch's) binding: one
+    warning, and every entry point goes on through its Python launcher."""
+    import types
+    import warnings
+
+    from fna2_amd import _capi
+
+    def missing(*a):
+        raise ImportError("undefined symbol")
+    monkeypatch.setattr("importlib.import_module", missing)
+    monkeypatch.setattr(_capi, "_native", None)
+    monkeypatch.setattr(_capi, "_native_missing", False)
+    t = types.SimpleNamespace(is_cuda=True)
+    with pytest.warns(RuntimeWarning, match="does not load.*Python launchers"):
+        assert F._native_fwd(t, t, t, None, None, None, 0.1, True) is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert F._native_bwd(t, t, t, t, None, None, None, t, t, 0.1, True) is None
+        assert _capi.native_or_none() is None
+    with pytest.raises(RuntimeError, match="build it"):
+        _capi.native()
+
+
+@pytest.mark.gpu
+def test_without_the_binding_every_entry_point(gpu, monkeypatch):
+    from fna2_amd import _capi, attention_fna2 as A
+    torch.manual_seed(0)
+    m = A.NaylisAttention(256, 4, rel_rank=16, max_seq_len=64, decode_graph_bias=True)
+    m = m.to(gpu).bfloat16().eval()
+    x, row = (torch.randn(2, s, 256, device=gpu).bfloat16() for s in (9, 1))
+
+    def calls():
+        c = A.StaticKVCache.empty(2, 4, 12, 64, 4, 16, device=gpu)
+        with torch.no_grad():
+            y, _ = m(x, past_kv=c, use_kv_cache=True)
+            z, _ = m(row, past_kv=c, use_kv_cache=True)
+        w, _ = m(x)
+        return (y, z, *torch.autograd.grad(w.sum(), list(m.parameters())))
+    a = calls()
+    monkeypatch.setattr(_capi, "_native", None)
+    monkeypatch.setattr(_capi, "_native_missing", True)
+    b = calls()
+    for i, (p, q) in enumerate(zip(a, b)):
+        # (the decode step's rows then come from the torch modules)
+        assert torch.equal(p, q) if i != 1 else Hp.rel_norm(p, q.double().cpu().numpy()) < 0.015
+
+
 CALLS = [  # dense or lengths, H, HKV, HG, D, R, causal, fp16
     ((2, 130), 8, 4, 6, 64, 24, True, False),
     ((1, 65), 4, 4, 0, 128, 0, False, False),
