@@ -123,6 +123,20 @@ Tensor bytes_on(size_t n, const Tensor& like) {
   return at::empty({(int64_t)std::max<size_t>(n, 1)}, like.options().dtype(at::kByte));
 }
 
+// The backward's workspace, with room for dK/dV items in chunks where the
+// library would use them (up to 512 MiB) and the memory is there: without
+// the room it runs the items whole.
+Tensor bwd_workspace(const fna2_problem& p, const Tensor& like) {
+  const size_t need = L.bwd_workspace_bytes(&p), chunks = L.bwd_split_bytes(&p);
+  if (chunks > 0) {
+    try {
+      return bytes_on(need + chunks, like);
+    } catch (const c10::OutOfMemoryError&) {
+    }
+  }
+  return bytes_on(need, like);
+}
+
 // The problem of an attention call, or false for the Python launcher.
 struct Call {
   fna2_problem p{};
@@ -282,8 +296,7 @@ std::optional<Grads> attn_bwd(const Tensor& dout, const Tensor& q, const Tensor&
     a.dr_k = view(drk, c.packed);
     a.d_graph_scale = dgs.data_ptr<float>();
   }
-  // (with room for dK/dV items in chunks, where the library would use them)
-  const Tensor ws = bytes_on(L.bwd_workspace_bytes(&c.p) + L.bwd_split_bytes(&c.p), q);
+  const Tensor ws = bwd_workspace(c.p, q);
   a.p = c.p;
   a.q = view(q, c.packed);
   a.k = view(k, c.packed);

@@ -250,9 +250,13 @@ def _run_fwd(prob, q, k, v, r_q, r_k, gs, out, lse, view, plan=None, plan_filled
 def _run_bwd(prob, tensors, view, plan=None):
     (dout, q, k, v, r_q, r_k, gs, out, lse, delta, dq, dk, dv, dr_q, dr_k, d_gs) = tensors
     L = _capi.lib()
-    # (with room for dK/dV items in chunks, where the library would use them)
-    ws = _workspace(lambda p: L.fna2_bwd_workspace_bytes(p) + L.fna2_bwd_split_bytes(p), prob,
-                    q.device)
+    # (with room for dK/dV items in chunks, where the library would use them
+    # and the memory is there: without the room it runs the items whole)
+    try:
+        ws = _workspace(lambda p: L.fna2_bwd_workspace_bytes(p) + L.fna2_bwd_split_bytes(p), prob,
+                        q.device)
+    except torch.OutOfMemoryError:
+        ws = _workspace(L.fna2_bwd_workspace_bytes, prob, q.device)
     ev = _events(KernelTimer.BWD)
     args = _capi.BwdArgs(prob, view(q), view(k), view(v), view(r_q), view(r_k), _ptr(gs),
                          view(out), view(lse), view(dout), view(delta), view(dq), view(dk),

@@ -172,3 +172,37 @@ def test_varlen_chunks(gpu, causal, D, R):
     for g, r in zip(got[:5], ref[:5]):
         assert not g[n:].any(), "rows outside every sequence"
         assert Hp.rel_norm(g[:n], r[:n]) < Hp.TOL_GRAD
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("path", ["native", "python"])
+def test_without_memory_for_chunks(gpu, monkeypatch, path):
+    """Where the chunks' partials do not fit in memory the items run whole:
+    the same gradients as with a workspace that has no room for chunks."""
+    import importlib
+    F = importlib.import_module("fna2_amd.flash_naylis_attn")
+    S, H, D, room = 4096, 8, 128, 40 << 20
+    prob = _problem(False, 1, S, S, H, 1, 0, D, 0, True)
+    assert _split_bytes(prob) > room
+    g = torch.Generator(device=gpu).manual_seed(5)
+    q, k, v, dout = (torch.randn(1, h, S, D, device=gpu, generator=g).bfloat16()
+                     for h in (H, 1, 1, H))
+    args = (q, k, v, None, None, None)
+    out, lse = F._fna2_forward(*args, 0.1, True)
+    if path == "python":
+        monkeypatch.setattr(F, "_native_bwd", lambda *a, **kw: None)
+    # the gradients (10 MiB) and the other scratch fit in `room`
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(gpu).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(gpu) + room) / total, gpu)
+    try:
+        got = F._fna2_backward(dout, *args, out, lse, 0.1, True)
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, gpu)
+    monkeypatch.setattr(F, "_native_bwd", lambda *a, **kw: None)
+    monkeypatch.setattr(F._capi.lib(), "fna2_bwd_split_bytes", lambda p: 0)
+    whole = F._fna2_backward(dout, *args, out, lse, 0.1, True)
+    for a, b in zip(got[:3], whole[:3]):
+        assert torch.equal(a, b)
