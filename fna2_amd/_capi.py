@@ -208,6 +208,7 @@ SIGNATURES = {
     "fna2_fwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(Problem)]),
     "fna2_bwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(Problem)]),
     "fna2_bwd_split_bytes": (ctypes.c_size_t, [ctypes.POINTER(Problem)]),
+    "fna2_key_groups": (ctypes.c_int, [ctypes.POINTER(Problem), ctypes.c_int]),
     "fna2_plan_bytes": (ctypes.c_size_t, [ctypes.POINTER(Problem)]),
     "fna2_fwd": (ctypes.c_int, [ctypes.POINTER(FwdArgs), ctypes.c_void_p]),
     "fna2_fwd_noalloc": (ctypes.c_int, [ctypes.POINTER(FwdArgs), ctypes.c_void_p]),

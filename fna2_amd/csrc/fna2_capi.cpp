@@ -161,34 +161,71 @@ BwdWs bwd_ws(const fna2_problem& p) {
   return w;
 }
 
-// Whether the forward's / dQ's query tiles are so few that the key groups'
-// variants (one workgroup of 8 to 16 waves per tile and CU) are the faster:
-// the tiles' longest key loop is then the kernel's time, and the groups cut
-// it, for some 3 us of combining.  That takes `min_keys` keys in the longest
-// tile, and at most one tile per CU -- two under the causal mask, whose tiles
-// differ in length.  Measured, us without -> with key groups, H heads x S:
-//   forward d64 r16  8x512 15.4 -> 15.3, 8x1024 23.8 -> 19.9, 16x2048 39.2 ->
-//     30.4, 16x4096 (512 tiles) 72.5 -> 59.7, non-causal 32x2048 (512) 54 -> 57,
-//     32x3001 (768) 62 -> 73
-//   forward d128 r32 8x256 14.8 -> 15.4, 8x512 21.3 -> 19.2, 16x2048 61 -> 43,
-//     32x1531 (384) 48.6 -> 39.5, 32x3001 (768) 101 -> 108
-//   dQ d64 r16  8x512 21.4 -> 20.9, 8x1024 34.2 -> 27.7, 16x2048 58.8 -> 41.9,
-//     32x2048 (512) 60 -> 55, non-causal 75 -> 82
-//   dQ d128 r32  8x512 25.8 -> 25.7, 8x1024 39.7 -> 36.5, 16x2048 69 -> 60,
-//     32x1531 (384) 58.6 -> 54.2, 32x3001 (768) 135 -> 154
-// (A varlen call counts its tiles by the tokens and half a tile per sequence
-// and takes the hinted length.)
+// Key groups of the forward's and dQ's kernels: with few query tiles, several
+// groups of four waves share a tile's keys (one workgroup of 8 to 16 waves per
+// tile and CU).  The tiles' longest key loop is then the kernel's time, and
+// the groups cut it, for some 3 us of combining: `min_keys` keys at least in
+// the longest tile.  Up to 256 tiles each has a CU to itself.  Up to 512 under
+// the causal mask, whose short tiles make a second round: it pays as long as
+// the long ones are few, `pairs` (sequence, head) pairs, each with one longest
+// tile.  Measured in bf16 (fp16 within 2%), us without -> with key groups, H
+// heads x S causal, nc: not:
+//   forward d64 r16   5x8x768 15.8 -> 15.3, 16x2048 32 -> 25, 32x1531 27 -> 26,
+//     32x2048 36 -> 35, 40x1024 19.8 -> 21.4, 10x8x768 17.9 -> 24.0; nc 5x8x768
+//     15.3 -> 15.6, 32x1024 19.3 -> 17.6.  r0 32x2048 30.9 -> 31.9, 24x2048 29.2
+//     -> 27.2; r64 32x2048 42 -> 40
+//   forward d128 r32  8x512 17.5 -> 16.3, 32x1531 43 -> 36.5, 32x2048 58 -> 52,
+//     37x1531 45.4 -> 45.5, 64x1024 34 -> 36; nc 5x8x768 23.8 -> 22.4, 16x2048
+//     53 -> 45.  r0 and r64 the same within 3%
+//   dQ d64 r16   32x1280 39 -> 33, 32x2048 58 -> 54, 48x1024 34 -> 36; nc 32x1024
+//     32 -> 29
+//   dQ d128 r32  34x1024 40 -> 38, 32x1531 55 -> 53.6, 32x2048 77.7 -> 78, 64x1024
+//     47 -> 54; nc 16x1024 36.8 -> 36.6, 8x2048 62 -> 57.5, 32x1024 39.7 -> 41,
+//     16x2048 67.8 -> 67.6; 768 keys: 0.7 to 2.5 us slower
+// A varlen call counts its tiles by the tokens and half a tile per sequence.
+// Its keys are what some sequence must have, the mean: max_seqlen_k is only a
+// bound, often a loose one, and short packs in these kernels lose a half (10
+// x 400, 8 heads: forward 20 -> 29 us).
 constexpr int kSplitCUs = 256;  // (a fixed figure: the answer depends on the arguments alone)
-bool few_tiles(const fna2_problem& p, int64_t min_keys) {
+
+// Tokens of a varlen pack's sequences, if they were of one length.
+int64_t mean_len(int64_t total, int64_t hint, int64_t batch) {
+  const int64_t mean = cdiv64(total, std::max<int64_t>(batch, 1));
+  return hint > 0 ? std::min(hint, mean) : mean;
+}
+
+bool few_tiles(const fna2_problem& p, int64_t min_keys, int64_t pairs) {
   int64_t tiles, keys;
   if (p.varlen) {
     tiles = cdiv64(p.total_q, kFwdBM) + p.batch / 2;
-    keys = p.seqlen_k > 0 ? std::min(p.seqlen_k, p.total_k) : p.total_k / std::max(p.batch, 1);
+    keys = mean_len(p.total_k, p.seqlen_k, p.batch);
   } else {
     tiles = (int64_t)p.batch * cdiv64(p.seqlen_q, kFwdBM);
     keys = p.causal ? std::min(p.seqlen_q, p.seqlen_k) : p.seqlen_k;
   }
-  return tiles * p.heads <= kSplitCUs * (p.causal ? 2 : 1) && keys >= min_keys;
+  tiles *= p.heads;
+  if (keys < min_keys) return false;
+  return tiles <= kSplitCUs ||
+         (p.causal && tiles <= 2 * kSplitCUs && tiles <= pairs * cdiv64(keys, kFwdBM));
+}
+
+int fwd_groups(const fna2_problem& p) {
+  const bool wide = p.head_dim == 128;
+  const int64_t min_keys = p.causal ? (wide ? 512 : 768) : (wide ? 768 : 1024);
+  if (!few_tiles(p, min_keys, wide || p.heads_graph > 0 ? 32 : 24)) return 1;
+  return fna2::fwd_key_groups(p.head_dim, fna2::padded_rank32(p.heads_graph, p.rank));
+}
+
+int dq_groups(const fna2_problem& p) {
+  const bool wide = p.head_dim == 128;
+  bool few = few_tiles(p, wide ? 1024 : 768, 32);
+  if (wide && !p.causal && few) {  // (every tile is a longest one)
+    const int64_t tiles =
+        p.heads * (p.varlen ? cdiv64(p.total_q, kDqBM) + p.batch / 2
+                            : (int64_t)p.batch * cdiv64(p.seqlen_q, kDqBM));
+    few = tiles <= kSplitCUs / 2 || few_tiles(p, 2048, 32);
+  }
+  return few ? fna2::dq_key_groups(p.head_dim, fna2::padded_rank32(p.heads_graph, p.rank)) : 1;
 }
 
 // dK/dV items in chunks.  The persistent dK/dV kernel deals (key tile, KV
@@ -534,6 +571,12 @@ size_t fna2_bwd_split_bytes(const fna2_problem* p) {
   return kv_split(*p).bytes;
 }
 
+int fna2_key_groups(const fna2_problem* p, int backward) {
+  if (!p) return FNA2_E_NULL;
+  FNA2_TRY(check_problem(*p));
+  return backward ? dq_groups(*p) : fwd_groups(*p);
+}
+
 size_t fna2_plan_bytes(const fna2_problem* p) {
   if (!p || check_problem(*p) != FNA2_OK) return 0;
   return plan_layout(*p).bytes;
@@ -593,9 +636,7 @@ int fwd_launch(const fna2_fwd_args* a, void* ws, hipStream_t stream) {
   }
   const int rpl = fna2::padded_rank32(K.p.H_G, K.p.R);
   if (!mark(a->events, 0, stream)) return FNA2_E_LAUNCH;
-  K.key_groups = few_tiles(p, p.head_dim == 128 ? 512 : 768)
-                     ? fna2::fwd_key_groups(p.head_dim, rpl)
-                     : 1;
+  K.key_groups = fwd_groups(p);
   if (fna2::launch_fwd(K, rpl, (int)g.fwd_grid, stream) != hipSuccess) return FNA2_E_LAUNCH;
   if (!mark(a->events, 1, stream)) return FNA2_E_LAUNCH;
   return FNA2_OK;
@@ -728,7 +769,7 @@ int fna2_bwd(const fna2_bwd_args* a, void* stream_ptr) {
     // (with a plan, one more row of workgroups than tiles can fill, so that
     // spare workgroups exist for the zeroing whatever the lengths)
     const int dq_grid = (int)g.dq_grid + (K.zero_uncovered ? p.heads : 0);
-    K.key_groups = few_tiles(p, 768) ? fna2::dq_key_groups(p.head_dim, rpl) : 1;
+    K.key_groups = dq_groups(p);
     if (rows_q(p) > 0 && fna2::launch_bwd_dq(K, rpl, dq_grid, stream) != hipSuccess)
       return FNA2_E_LAUNCH;
     if (!mark(a->events, 1, stream) || !mark(a->events, 2, stream)) return FNA2_E_LAUNCH;

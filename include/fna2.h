@@ -331,6 +331,10 @@ size_t fna2_bwd_workspace_bytes(const fna2_problem* p);
  * dK/dV items that would leave CUs idle in chunks (the same sums, fp32
  * partials added in a fixed order); with less it runs them whole. */
 size_t fna2_bwd_split_bytes(const fna2_problem* p);
+/* Groups of waves that share a query tile's keys in this problem's forward
+ * (backward = 0) or dQ kernel (1): 1, or more where its tiles are few.  Host
+ * only; the status of a problem that is refused. */
+int fna2_key_groups(const fna2_problem* p, int backward);
 
 /* Bytes of a plan (the varlen tile lists of the forward and the backward:
  * device-built, so no host synchronisation); 0 in dense mode.  No
