@@ -236,16 +236,25 @@ int dq_groups(const fna2_problem& p) {
 // write fp32 partials to the workspace for a reduction kernel.  The rule
 // compares, in blocks (32 queries against a key tile), the longest chunk and
 // a CU's share with what entering a chunk costs (kEnter) and the reduction
-// (its launch and the partials written and read); in varlen mode, where the
-// host does not know the lengths, it takes the pack as total_k / max_seqlen
-// sequences of the hinted length.
+// (its launch and the partials written and read); without the causal mask all
+// chunks are alike, so the CUs also go through them in whole rounds.  In
+// varlen mode the host does not know the lengths, and max_seqlen is only a
+// bound, often a loose one: chunks that the real items do not need cost up to
+// their own time (32 x 128, 8/4 heads, d 64, max_seqlen 4096: backward 39 ->
+// 75 us).  So the best split is taken for a pack of max_seqlen's sequences,
+// of those that cost a pack of its mean length nothing: up to 1.1 times the
+// whole items by this estimate, in 2 to 8 chunks (of 33 such packs measured
+// none was slower; of 27 between 1.2 and 1.4, 12 were, and 16 chunks at 1.1).
 //
 // Measured (dK/dV and its reduction, us, whole items -> the rule's chunks):
 // B2 H16/4 L1531 d128 fp16 238 -> 88 (chunks of 1/2: 138, 1/4: 86, 1/8: 96,
 // 1/16: 120), B1 H8/4 L512 d64 51 -> 24, B1 H32/8 L1024 d128 158 -> 60, B1
-// H8/4 L8192 d128 580 -> 355.  Where the rule keeps them whole: B1 H16 L2048
-// d128 (256 items) 85 whole, 82 in halves, 104 in quarters; B1 H8 L128 15
-// against 18.
+// H8/4 L8192 d128 580 -> 355; packs of one long sequence, max_seqlen exact or
+// not, the backward: [1191, 6 x ~117] H16/4 d128 233 -> 110, [7083, 3 x ~1150]
+// H12/4 d64 not causal 1142 -> 833.  Where the rule keeps them whole: B1 H16
+// L2048 d128 (256 items) 85 whole, 82 in halves, 104 in quarters; B1 H8 L128
+// 15 against 18; B3 L3209 H12/4 d64 not causal (156 items) 350 whole, 408 in
+// halves.
 struct KvSplit {
   int log2 = 0;
   int64_t tiles = 0;
@@ -259,39 +268,50 @@ KvSplit kv_split(const fna2_problem& p) {
   if (p.batch <= 0 || g.kv_grid <= 0) return best;
   const int bn = kv_tile(p);
   const int group = p.heads / p.heads_kv;
-  int64_t lq, lk, nseq;
-  if (p.varlen) {
-    lk = p.seqlen_k > 0 && p.seqlen_k < p.total_k ? p.seqlen_k : p.total_k;
-    lq = p.seqlen_q > 0 && p.seqlen_q < p.total_q ? p.seqlen_q : p.total_q;
-    nseq = lk > 0 ? std::max<int64_t>(p.total_k / lk, 1) : 1;
-  } else {
-    lk = p.seqlen_k;
-    lq = p.seqlen_q;
-    nseq = p.batch;
-  }
-  const int64_t qb = cdiv64(lq, kKvBM), kt = cdiv64(lk, bn), lo = p.causal ? bn / kKvBM : 0;
-  if (qb <= 0 || kt <= 0) return best;
-  // blocks of one sequence and head: sum over its key tiles of qb - lo t
-  const int64_t seen = lo > 0 ? std::min<int64_t>(kt, cdiv64(qb, lo)) : kt;
-  const int64_t per_head = seen * qb - lo * (seen * (seen - 1) / 2);
-  const int64_t items = nseq * kt * p.heads_kv;
-  const int64_t total = nseq * p.heads * per_head;
-  const int64_t longest = (int64_t)group * qb;
   const int64_t rpl = fna2::padded_rank32(p.heads_graph, p.rank);
-  const int64_t cut = p.varlen ? std::min<int64_t>(g.kv_tiles, cdiv64(p.total_k, bn) + 8)
-                               : g.kv_tiles;
+  // The work as nseq sequences of lq x lk: items, blocks in all and of the
+  // longest item.
+  struct Work {
+    int64_t kt = 0, items = 0, total = 0, longest = 0;
+  };
+  auto work = [&](int64_t lq, int64_t lk, int64_t nseq) {
+    Work w;
+    const int64_t qb = cdiv64(lq, kKvBM), lo = p.causal ? bn / kKvBM : 0;
+    w.kt = cdiv64(lk, bn);
+    // blocks of one sequence and head: sum over its key tiles of qb - lo t
+    const int64_t seen = lo > 0 ? std::min<int64_t>(w.kt, cdiv64(qb, lo)) : w.kt;
+    w.items = nseq * w.kt * p.heads_kv;
+    w.total = nseq * p.heads * (seen * qb - lo * (seen * (seen - 1) / 2));
+    w.longest = (int64_t)group * qb;
+    return w;
+  };
   constexpr double kEnter = 4, kLaunch = 5, kBytesPerBlock = 4e6;
-  auto cost = [&](int log2) {
+  auto cost = [&](const Work& w, int log2) {
     const int64_t n = (int64_t)1 << log2;
-    const double len = (double)std::max<int64_t>(cdiv64(longest, n), log2 ? fna2::kKvMinChunk : 1);
-    const double chunks = std::min((double)items * n, std::max((double)total / fna2::kKvMinChunk,
-                                                               (double)items));
-    double t = std::max(len + kEnter, (total + kEnter * chunks) / kSplitCUs);
-    if (log2 > 0)
-      t += kLaunch + chunks * bn * (2 * p.head_dim + rpl) * 8.0 / kBytesPerBlock;
+    const int64_t len = std::max<int64_t>(cdiv64(w.longest, n), log2 ? fna2::kKvMinChunk : 1);
+    const double chunks = std::min((double)w.items * n,
+                                   std::max((double)w.total / fna2::kKvMinChunk, (double)w.items));
+    double t = std::max(len + kEnter, (w.total + kEnter * chunks) / kSplitCUs);
+    if (!p.causal)
+      t = std::max(t, cdiv64(w.items * cdiv64(w.longest, len), kSplitCUs) * (len + kEnter));
+    if (log2 > 0) t += kLaunch + chunks * bn * (2 * p.head_dim + rpl) * 8.0 / kBytesPerBlock;
     return t;
   };
-  double least = 0.9 * cost(0);
+  const int64_t lq = p.varlen ? mean_len(p.total_q, p.seqlen_q, p.batch) : p.seqlen_q;
+  const int64_t lk = p.varlen ? mean_len(p.total_k, p.seqlen_k, p.batch) : p.seqlen_k;
+  const Work even = work(lq, lk, p.batch);
+  Work hinted = even;
+  if (p.varlen && p.seqlen_q > lq && p.seqlen_k > lk) {
+    const int64_t hk = std::min(p.seqlen_k, p.total_k);
+    hinted = work(std::min(p.seqlen_q, p.total_q), hk, std::max<int64_t>(p.total_k / hk, 1));
+  }
+  if (even.total <= 0) return best;
+  // (a whole item after the chunks is the last to end: in a pack of equal
+  // lengths every tile is cut, in others the shortest may stay whole)
+  const int64_t cut =
+      std::min(g.kv_tiles, std::max(p.batch * even.kt, p.varlen ? cdiv64(p.total_k, bn) + 8 : 0));
+  double least = 0.9 * cost(hinted, 0);
+  const double whole = cost(even, 0);
   for (int log2 = 1; log2 <= 4; ++log2) {
     KvSplit s;
     s.log2 = log2;
@@ -304,7 +324,8 @@ KvSplit kv_split(const fna2_problem& p) {
     if (s.tiles <= 0 || (s.tiles * p.heads_kv) << log2 > kMaxGrid) continue;
     s.drk_part = align_up((size_t)(s.tiles * kv));
     s.bytes = s.drk_part + align_up((size_t)(s.tiles * dr));
-    const double t = cost(log2);
+    if (cost(even, log2) > (log2 < 4 && hinted.longest > even.longest ? 1.1 : 0.9) * whole) continue;
+    const double t = cost(hinted, log2);
     if (t < least) {
       least = t;
       best = s;

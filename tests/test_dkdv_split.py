@@ -148,7 +148,7 @@ def test_dense_chunks(gpu, case):
 @pytest.mark.parametrize("D,R", [(64, 16), (128, 32)])
 def test_varlen_chunks(gpu, causal, D, R):
     """One long sequence beside short and empty ones, tokens outside every
-    sequence, a vanilla head; the long tiles in chunks, the short ones whole."""
+    sequence, a vanilla head; every tile in chunks as long as it has blocks."""
     import importlib
     F = importlib.import_module("fna2_amd.flash_naylis_attn")
     lens, H, HKV, HG = [40, 0, 1300, 17, 129], 4, 2, 3
@@ -206,3 +206,70 @@ def test_without_memory_for_chunks(gpu, monkeypatch, path):
     whole = F._fna2_backward(dout, *args, out, lse, 0.1, True)
     for a, b in zip(got[:3], whole[:3]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("D,R", [(64, 16), (128, 32)])
+def test_whole_items_after_the_chunks(gpu, causal, D, R):
+    """A pack with more key tiles than the rule cuts: the longest in chunks,
+    the last of the short ones whole, in one launch."""
+    import importlib
+    F = importlib.import_module("fna2_amd.flash_naylis_attn")
+    lens, H, HKV, HG = [2000] + [33] * 29, 8, 1, 6
+    total, N, bn = sum(lens), len(lens), 256 if D == 64 else 128
+    q, k, v, rq, rk, gs, dout, cu, _ = Hp.make_varlen(lens, H, D, HKV, HG, R, seed=D)
+    dev = [t.to(gpu) for t in (q, k, v, rq, rk, gs, dout, cu)]
+    dq, dk, dv, drq, drk, dgs, ddo, dcu = dev
+    scale = 1 / math.sqrt(D)
+    prob = F._problem(True, N, 2000, 2000, total, total, H, HKV, HG, D, R, causal, scale, dcu, dcu)
+    cut = max(N * -(-(total // N) // bn), -(-total // bn) + 8)
+    assert cut < sum(-(-n // bn) for n in lens)
+    # partials of `cut` tiles: dK | dV of 2^l chunks, dRk of 2^l + group - 1
+    assert _split_bytes(prob) in [cut * bn * 4 * ((2 * D << l) + (H + (1 << l) - 1) * 32)
+                                  for l in range(1, 5)]
+    print("whole after chunks", D, R, causal, flush=True)
+    out, lse = F._fna2_forward_varlen(dq, dk, dv, drq, drk, dgs, dcu, dcu, 2000, 2000, scale,
+                                      causal)
+    run = lambda: F._fna2_backward_varlen(ddo, dq, dk, dv, drq, drk, dgs, out, lse, dcu, dcu, 2000,
+                                          2000, scale, causal)
+    got, again = run(), run()
+    lib = F._capi.lib()
+    keep, native = lib.fna2_bwd_split_bytes, F._native_bwd
+    try:
+        lib.fna2_bwd_split_bytes, F._native_bwd = lambda p: 0, lambda *a, **kw: None
+        whole = run()
+    finally:
+        lib.fna2_bwd_split_bytes, F._native_bwd = keep, native
+    torch.cuda.synchronize()
+    for a, b, c in zip(got, whole, again):
+        assert torch.equal(a, c), "not reproducible"
+        assert Hp.rel_norm(a, b.double().cpu().numpy()) < 4e-3  # (as in test_dense_chunks)
+    for i in (1, 2):  # the whole items' keys: the last seven short sequences
+        assert torch.equal(got[i][-33:], whole[i][-33:])
+    _, _, ref = Hp.oracle_fwd_bwd(q, k, v, rq, rk, gs, dout, scale, causal, cu.numpy(), cu.numpy())
+    Hp.check_grads(got[:5], ref[:5])
+
+
+def test_split_rule_does_not_trust_max_seqlen():
+    """A loose max_seqlen (the token count, none) does not cut the items of
+    short sequences."""
+    for hint in (0, 128, 768, 4096):
+        p = _problem(True, 32, hint, hint, 8, 4, 8, 64, 16, True, None)
+        p.total_q = p.total_k = 4096
+        p.cu_seqlens_q = p.cu_seqlens_k = 1 << 20
+        assert _split_bytes(p) == 0
+    # one long sequence is known by its mean
+    p = _problem(True, 2, 0, 0, 8, 4, 8, 64, 16, True, None)
+    p.total_q = p.total_k = 4096
+    p.cu_seqlens_q = p.cu_seqlens_k = 1 << 20
+    assert _split_bytes(p) > 0
+
+
+def test_equal_chunks_go_in_whole_rounds():
+    """Without the mask the chunks are alike: 312 halves of 156 items are two
+    rounds of 256 CUs, no shorter than the items whole."""
+    assert _split_bytes(_problem(False, 3, 3209, 3209, 12, 4, 12, 64, 16, False)) == 0
+    # 104 items: one round of halves
+    halves = 2 * 13 * 4 * 256 * 4 * ((2 * 64 << 1) + (3 + (1 << 1) - 1) * 32)
+    assert _split_bytes(_problem(False, 2, 3209, 3209, 12, 4, 12, 64, 16, False)) == halves
