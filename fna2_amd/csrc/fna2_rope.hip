@@ -39,7 +39,7 @@ constexpr int kRopePasses = 4;  // row passes whose loads are in flight together
 // weights in registers).  Passes in flight per wave, 16-bit and fp32: with
 // 16-bit rows a second one no longer fits four waves' registers (c3 pack: 90.6
 // us; two passes at three waves 98, four at two 109; before, 104.  fp32, 6000
-// tokens: two passes 66, one 73; before, 84).
+// tokens: two passes 66, one 73; before, 84.  fp16, c3 pack: 90; before, 108).
 constexpr int kBwdOcc = 4;
 template <int DT>
 constexpr int kBwdPasses = DT == kRopeF32 ? 2 : 1;
@@ -420,6 +420,11 @@ __global__ __launch_bounds__(64 * kRopeWaves, kBwdOcc) void rope_norm_bwd_kernel
           // (a lane past the rows holds zeros; every lane joins the sums)
           ss = row_sum(ss, L.lpr);
           tw = row_sum(tw, L.lpr);
+          // (fp16: the products below stay behind the sums.  Begun ahead of
+          // them, they spilled 9 registers: 16384 tokens, d128 91.0 -> 90.1
+          // us, 6000 35.2 -> 34.5, 3000 26.5 -> 26.8.  In bf16 they spill
+          // one, outside the loop; there the order costs 1 to 3%.)
+          if constexpr (DT == kRopeF16) asm volatile("" : "+v"(ss));
           if (has_w) {
             const float rr = rsqrtf(ss * inv_d + P.eps);
             const float k3 = rr * rr * rr * tw * inv_d;

@@ -11,6 +11,11 @@ to the next ``s_barrier``, no instruction outside inline assembly reads or
 writes the load's destination registers (a copy or spill there would see
 the register before the data lands).  This test rebuilds the kernel to
 assembly with the library's own flags and walks every path.
+
+``test_rotary_kernels_do_not_spill``: the rotary kernels are bound by their
+loads in flight, and fit the waves per SIMD that they are built for without
+scratch memory in every type (but for one register of the norm backward in
+bf16, kept outside its loop).
 """
 import os
 import re
@@ -105,3 +110,20 @@ def test_dkdv_inplace_row_loads_untouched_until_barrier(tmp_path):
     loads, bad = inplace_violations(out.read_text())
     assert loads >= 6 * 18, loads  # every kernel variant has its row loads
     assert not bad, bad[:5]
+
+
+@pytest.mark.skipif(not (shutil.which("hipcc") or os.path.exists("/opt/rocm/bin/hipcc")),
+                    reason="hipcc not available")
+def test_rotary_kernels_do_not_spill(tmp_path):
+    from fna2_amd import build as B
+    out = tmp_path / "rope.s"
+    cmd = [B.HIPCC, *B.COMMON, "--cuda-device-only", "-S", str(B.CSRC / "fna2_rope.hip"),
+           "-o", str(out)]
+    subprocess.run(cmd, check=True, capture_output=True)
+    asm = out.read_text()
+    names = re.findall(r"^\s+\.symbol:\s+(\S*rope\S*)\.kd", asm, re.M)
+    spills = re.findall(r"^\s+\.vgpr_spill_count:\s+(\d+)", asm, re.M)
+    scratch = re.findall(r"^\s+\.private_segment_fixed_size:\s+(\d+)", asm, re.M)
+    assert len(names) == len(spills) == len(scratch) == 10
+    left = {n: (int(a), int(b)) for n, a, b in zip(names, spills, scratch) if a != "0" or b != "0"}
+    assert all("rope_norm_bwd_kernelILi1E" in n and v <= (1, 8) for n, v in left.items()), left
