@@ -143,6 +143,148 @@ def test_attention_bits(gpu, call, strided):
         assert torch.equal(p, s)
 
 
+def _through_python(fn, monkeypatch):
+    """fn as if the binding were not there."""
+    from fna2_amd import _capi
+    with monkeypatch.context() as m:
+        m.setattr(_capi, "native_or_none", lambda: None)
+        return fn()
+
+
+def _same(a, b):
+    for x, y in zip(a, b):
+        assert (x is None) == (y is None)
+        assert x is None or (x.stride() == y.stride() and torch.equal(x, y))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=str)
+@pytest.mark.parametrize("D,H,HKV,norms", [(64, 8, 2, "qk"), (128, 3, 3, "q"), (128, 4, 1, "")])
+def test_rope_bits(gpu, native, monkeypatch, dtype, D, H, HKV, norms):
+    """The rotation and its backward, into new tensors and into slices of a
+    wider one, with rows outside every sequence."""
+    from fna2_amd import rope as Ro
+    g = torch.Generator(device=gpu).manual_seed(D + H)
+    T, cu = 201, torch.tensor([3, 70, 70, 195], dtype=torch.int32, device=gpu)
+    mk = lambda *s: torch.randn(*s, generator=g, device=gpu).to(dtype)
+    wide = mk(T, H + HKV, D)
+    q, k = wide[:, :H], wide[:, H:]
+    dq, dk = mk(T, H, D), mk(T, HKV, D)
+    inv = 1.0 / 10000 ** (torch.arange(0, D, 2, device=gpu) / D)
+    nq = 1 + 0.2 * mk(D) if "q" in norms else None
+    nk = 1 + 0.2 * mk(D) if "k" in norms else None
+    assert native.rope_fwd(q, k, cu, inv, 1, nq, nk, 1e-6) is not None
+    for sign in (1, -1):
+        fwd = lambda: Ro.rope_varlen_raw(q, k, cu, inv, sign, nq, nk, 1e-6)
+        _same(fwd(), _through_python(fwd, monkeypatch))
+    slabs = []
+
+    def bwd(given=False):
+        to = {}
+        if given:
+            slabs.append(torch.zeros(T, H + HKV + 1, D, device=gpu, dtype=dtype))
+            to = dict(dq=slabs[-1][:, :H], dk=slabs[-1][:, H:H + HKV])
+        return Ro.rope_varlen_bwd(dq, dk, q, k, cu, inv, 1, nq, nk, 1e-6, **to)
+    one = bwd()
+    _same(one, _through_python(bwd, monkeypatch))
+    given = lambda: bwd(True)
+    two = given()
+    _same(two, _through_python(given, monkeypatch))
+    assert torch.equal(slabs[0], slabs[1]) and not slabs[0][:, -1].any()
+    for x, y in zip(one, two):
+        assert x is None or torch.equal(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,HKV,HG,D,R,L", [(3, 8, 2, 6, 64, 24, 700), (2, 4, 4, 0, 128, 0, 33),
+                                               (5, 8, 1, 8, 128, 16, 1000)])
+def test_decode_bits(gpu, native, monkeypatch, B, H, HKV, HG, D, R, L):
+    """The decode: all rows or ragged ones, a cache in either order, q as
+    [B, H, D] or [B, H, 1, D], graph_scale in fp32 or bf16, split or whole."""
+    from fna2_amd.decode import flash_naylis_decode
+    g = torch.Generator(device=gpu).manual_seed(B + L)
+    mk = lambda *s: torch.randn(*s, generator=g, device=gpu).bfloat16()
+    q, k, v = mk(B, 1, H, D).transpose(1, 2), mk(B, L, HKV, D).transpose(1, 2), mk(B, HKV, L, D)
+    rq, rk = (mk(B, HG, 1, R), mk(B, HG, L, R)) if HG else (None, None)
+    gs = 1 + 0.5 * mk(HG) if HG else None
+    seq = torch.tensor([(17 + 211 * i) % (L + 1) for i in range(B)], dtype=torch.int32, device=gpu)
+    row = lambda t, flat: t if t is None or not flat else t[:, :, 0]
+    for flat in (True, False):
+        for lens in (None, seq):
+            for scale in (gs, gs if gs is None else gs.float()):
+                for n in (0, 1, 3):
+                    run = lambda: flash_naylis_decode(row(q, flat), k, v, row(rq, flat), rk, scale,
+                                                      cache_seqlens=lens, num_splits=n,
+                                                      return_lse=True)
+                    _same(run(), _through_python(run, monkeypatch))
+    assert native.decode(q, k, v, rq, rk, gs, 0.1, seq, 0) is not None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("path", ["native", "python"])
+def test_calls_run_on_the_current_stream(gpu, native, monkeypatch, path):
+    """Every entry point on a stream of its own: its inputs are written there
+    behind a wait of some milliseconds, so a launch on any other stream would
+    read the zeros that they held before."""
+    from fna2_amd import _capi, attention_fna2 as A, decode as De, rope as Ro
+    if path == "python":
+        monkeypatch.setattr(_capi, "native_or_none", lambda: None)
+    torch.manual_seed(0)
+    H, HKV, D, R, S = 4, 2, 64, 16, 300
+    rnd = lambda *s: torch.randn(*s, device=gpu).bfloat16()
+    dense = [rnd(2, h, S, f) for h, f in ((H, D), (HKV, D), (HKV, D), (H, R), (H, R))]
+    gs, dout = torch.ones(H, device=gpu), rnd(2, H, S, D)
+    pack = [t.transpose(1, 2).reshape(2 * S, *t.shape[1:2], t.shape[3]) for t in dense]
+    pdout = dout.transpose(1, 2).reshape(2 * S, H, D)
+    cu = torch.tensor([0, S, 2 * S], dtype=torch.int32, device=gpu)
+    inv, w = torch.ones(D // 2, device=gpu), 1 + 0.1 * rnd(D)
+    m = A.NaylisAttention(256, H, rel_rank=R, max_seq_len=64).to(gpu).bfloat16().eval()
+    x = rnd(2, 1, 256)
+
+    def train(*a):
+        leaves = [t.detach().requires_grad_(True) for t in a[:-1]]
+        out = F.flash_naylis_attn(*leaves, is_causal=True)
+        return (out, *torch.autograd.grad(out, leaves, a[-1]))
+
+    def fwd_bwd_varlen(q, k, v, rq, rk, g, do):
+        out, lse = F._fna2_forward_varlen(q, k, v, rq, rk, g, cu, cu, S, S, 0.125, True)
+        return (out, lse, *F._fna2_backward_varlen(do, q, k, v, rq, rk, g, out, lse, cu, cu, S, S,
+                                                   0.125, True))
+
+    def step(row, k, v):
+        c = A.StaticKVCache.empty(2, H, 8, D, device=gpu)
+        with torch.no_grad():
+            c.append(k, v)
+            y, _ = m(row, past_kv=c, use_kv_cache=True)
+        return y, c.k[:, :, :4], c.v[:, :, :4]
+    calls = [
+        ("train", train, (*dense, gs, dout)),
+        ("varlen", fwd_bwd_varlen, (*pack, gs, pdout)),
+        ("decode", lambda q, *a: De.flash_naylis_decode(q, *a, return_lse=True),
+         (dense[0][:, :, 0], dense[1], dense[2], dense[3][:, :, 0], dense[4], gs)),
+        ("rope", lambda q, k, a, b: Ro.rope_varlen_raw(q, k, cu, inv, 1, a, b, 1e-6),
+         (pack[0], pack[1], w, w)),
+        ("rope_bwd", lambda *a: Ro.rope_varlen_bwd(*a[:4], cu, inv, 1, *a[4:], 1e-6),
+         (pdout, pack[1], pack[0], pack[1], w, w)),
+        ("step", step, (x, rnd(2, H, 3, D), rnd(2, H, 3, D))),
+    ]
+    side = torch.cuda.Stream()
+    for name, fn, args in calls:
+        print(path, name, flush=True)
+        ref = fn(*args)
+        bufs = [torch.zeros_like(t) for t in args]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(5_000_000)
+            for b, t in zip(bufs, args):
+                b.copy_(t)
+            got = fn(*bufs)
+            waiting = not side.query()
+        side.synchronize()
+        assert waiting or path == "python", "the call waited for its stream"
+        _same(got, ref)
+
+
 @pytest.mark.gpu
 def test_calls_left_to_the_python_launcher(gpu):
     q, k, v, rq, rk, gs, dout = [t.to(gpu) for t in Hp.make_dense(1, 4, 64, 64, 4, 4, 16)]
