@@ -805,9 +805,9 @@ __device__ __forceinline__ void dkdv_body(const BwdParams& P) {
       }
     };
     // SPLIT: a wave's fp32 accumulator tile (32 features x 32 keys) as it
-    // lies in the registers, 16 bytes per lane: tile `t` of the slice's
-    // part_tiles(D) (dK, then dV) in the chunk's slot, or of its RPL / 32 in
-    // a dRk slot.
+    // lies in the registers, 16 bytes per lane: one of the
+    // slice's 2 NDB (dK, then dV) in the chunk's slot, or of its NRB in a dRk
+    // slot.
     auto put_tile = [&](float* base, const f32x16& a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)

@@ -323,7 +323,7 @@ __device__ __forceinline__ void decode_body(const DecodeParams& P) {
 // One workgroup per (sequence, head) combines the splits' partial results.
 // A row of D fp32 values is 16 bytes for each of D / 4 lanes, so a wave reads
 // 256 / D splits at once and the four waves 4 of those, kMergeAhead deep:
-// the loads of 40 splits are all in flight together.  (One wave per row,
+// the loads of 32 splits (64 at d = 64) are all in flight together.  (One wave per row,
 // one split after the other, was a chain of nsplit loads: 7.0 us for 20
 // splits of 128 rows; decode and merge of 4 sequences of 2500 rows, H32/8
 // d128: 17.3 -> 12.5 us.)  The sum's order depends on nsplit alone.

@@ -88,12 +88,20 @@ def test_rows_against_the_formula(gpu, case):
             x = x * cos.double() + h * sin.double()
         return x
 
-    # two roundings to bf16 (2^-9 each of values up to |x| + |partner|)
+    # roundings to bf16, 2^-8 of the value each: the normalised x and its
+    # partner before the rotation (|x cos| + |partner sin|), then the result
     for got, x, w, eps in ((out[:, :, None], q, wq, 1e-6), (at(kc), k, wk, 1e-3)):
         r = ref(x, w, eps)
-        lim = 2 ** -8 * (ref(x.abs(), None if w is None else w.abs(), eps).abs() * 0 +
-                         r.abs().amax(-1, keepdim=True) * 2 + 1e-6)
-        assert ((got.double() - r).abs() <= lim).all()
+        lim = torch.zeros_like(r)
+        if norm:
+            n = x.double()
+            n = n * torch.rsqrt(n.square().mean(-1, keepdim=True) + eps) * w.double()
+            part = torch.cat((n[..., D // 2:], n[..., :D // 2]), -1)
+            lim += n.abs() if cos is None else (n * cos.double()).abs() + (part * sin.double()).abs()
+        if rope:
+            lim += r.abs()
+        # (1 + 2^-6: the first roundings within the second, and the fp32 sums)
+        assert ((got.double() - r).abs() <= 2 ** -8 * (1 + 2 ** -6) * lim).all()
     assert torch.equal(at(vc), v)
     if HG:
         assert torch.equal(at(rc), rk)

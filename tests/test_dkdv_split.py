@@ -136,7 +136,7 @@ def test_dense_chunks(gpu, case):
             continue
         assert torch.equal(a, c), "not reproducible"
         # the same fp32 terms in another order, rounded once to 16 bits
-        # (2^-9 of a value, half the values at most one step apart)
+        # (at most 2^-8 of a value on each side, and the same for most)
         assert Hp.rel_norm(a, b.double().cpu().numpy()) < 4e-3
     q, k, v, rq, rk, gs, dout = ins
     _, _, ref = Hp.oracle_fwd_bwd(q, k, v, rq, rk, gs, dout, scale, causal)
