@@ -1013,7 +1013,6 @@ namespace {
 // (a fixed figure, so that the split count and the workspace size are a
 // function of the arguments alone).
 constexpr int kDecodeCUs = 256;
-constexpr int64_t kDecodeFewWaves = 2 * kDecodeCUs;
 constexpr int64_t kOff31 = ((int64_t)1 << 31) - 16;  // buffer-offset bound
 
 int dec_group(const fna2_decode_args& a) { return a.heads / a.heads_kv; }
@@ -1038,46 +1037,96 @@ struct DecSplit {
   int n = 1, keys = 32;
 };
 
-// The library's split count.  The waves that run at once are at most four per
-// CU (what reads at the full rate) and what the ring's LDS leaves room for:
-// one round of them, since a second, partly filled one is waited for by
-// half the chip -- and at least four steps a split.  Where the lengths differ
-// (`ragged`) the longest sequences would be the whole time: four splits at
-// least, eight where a round holds fewer than four (several rounds then, whose
-// later waves level the lengths).  Measured, decode and merge, us, two rounds
-// (the rule before) -> this one, ragged as the mean of three draws:
-//   64 sequences x 4096, H16 R32      403 -> 397, ragged 264 -> 243 (4: 244)
-//   64 x 4096, H32/8 R32 (3 a CU)     285 -> 278, ragged 211 -> 191 (4: 182)
-//   16 x 2048, H16 R32                54.9 -> 55.2, ragged 41.4 -> 36.6
-//   24 x 5000, H16 R32                211 -> 192, ragged 133 -> 124 (4: 127)
-//   15 x 5065, H32                    216 -> 212, ragged 146 -> 147 (4: 156)
-//   48 x 3000, H16 d64                108 -> 102, ragged 69 -> 68 (4: 71)
-//   20 x 6000, H32/8                  100 -> 91, ragged 57 -> 54
-// Few units: a split's steps are a chain of load latencies that nothing else
-// hides, so down to one step each as long as the waves stay few (two per CU;
-// more and the merge and the waves' own start outweigh it).  Up to two steps
-// a second launch costs more than it saves.  (Four-step splits -> the rule's:
-// B2 H8/4 L496 d128 13.0 -> 9.0, B1 H16 L200 d64 10.0 -> 7.7, B1 H32/8 L4096
-// d128 10.7 -> 9.7; B1 H8 L64 6.4 whole, 8.3 in two; B4 H32/8 L2500: 20 splits
-// (640 waves) 12.2, 40 15.8.)
+// The library's split count.
+//
+// Small caches: the least estimated time over the counts that differ.  A
+// wave walks its split's 32-key steps, each a chain of latencies (`step`,
+// longer with the rank tile and with more waves on the CU), behind its own
+// start (`kStart`).  As many waves run at once as the ring's LDS leaves room
+// for, so they come in rounds, the last partly filled, each as long as its
+// chain or as reading its share of the cache takes.  More than one split adds
+// the merge (`kMerge` and its partials).  Where the lengths differ (the host
+// does not know them) the last round holds a longest split; the others, and
+// the bytes, count two thirds.
+// Large ones (kDecodeLarge): the rate follows the waves in flight, up to four
+// per CU, so one round of them as full as whole splits make it, of at least
+// four steps; with differing lengths (kDecodeRagged) up to eight rounds, which
+// level them, of eight steps, while the partials are few.
+//
+// Fitted to 388 calls of 1 to 128 sequences, 4 to 32 heads and 33 to 40,000
+// rows, timed behind a full queue at up to 20 counts each (us).  Against the
+// best count of each, mean and most: small caches 1.006 and 1.14, large ones
+// 1.02 and 1.10, ragged 1.03 and 1.13.  (One round of waves and one-step
+// splits for few units, at any size: 1.056 and 1.9 for the small, 1.05 and
+// 1.18 for the large and ragged; two rounds: 1.16 and 1.9, 1.07 and 1.3.)
+// What those missed:
+//   up to four to six steps a second launch costs more than it saves: B4 H4/1
+//     d64 L84 5.2 whole, 7.4 in three; B2 H8/2 d128 r16 L73 8.0, 9.9
+//   waves just past a round: B3 H32 d128 L7267 9 splits 65, 12 80; B118 H4/2
+//     d128 r8 L305 4 splits 15.1, 5 19.2
+//   ragged lengths in full rounds anyway: B97 H32 d128 L304 59 whole, 76 in
+//     three
+//   large and ragged: B26 H8 d128 r32 L23182 4 splits 388, 32 341
+// The lines: equal lengths, 300 to 600 MB, the estimate's counts 1.04 times
+// the best, one round 1.01 (B20 H32/8 L6000, 491 MB: 104, 90); below the 256
+// MB that the last cache level holds 1.011 and 1.016.  Differing lengths, 350
+// to 600 MB: the estimate 1.03, the rounds 1.10; above, 1.055 and 1.03.
+constexpr double kDecodeLarge = 256e6, kDecodeRagged = 600e6;
 DecSplit dec_split(const fna2_decode_args& a, bool ragged) {
   DecSplit s;
   const int64_t L = a.max_seqlen_k;
   if (L <= 0) return s;
+  const int64_t steps = cdiv64(L, 32);
   int64_t n = a.num_splits;
   if (n <= 0) {
-    const int64_t units = std::max<int64_t>((int64_t)a.batch * a.heads_kv, 1);
     const int rc = std::max(dec_rc(a), 0);
-    const int per_cu = std::max(1, (160 * 1024) / (fna2::kDecodeStages *
-                                                   fna2::decode_stage_bytes(a.head_dim, rc)));
-    n = (int64_t)kDecodeCUs * std::min(per_cu, 4) / units;
-    if (ragged) n = std::max<int64_t>(n, n < 4 ? 8 : 4);
-    n = std::min<int64_t>(n, cdiv64(L, 128));
-    if (L > 64) n = std::max<int64_t>(n, std::min<int64_t>(kDecodeFewWaves / units, cdiv64(L, 32)));
-    n = std::max<int64_t>(std::min<int64_t>(n, 64), 1);
-    if (L <= 64) n = 1;
+    // (one byte less: the full 160 KB do not all go to workgroups)
+    const int per_cu = std::max(
+        1, (160 * 1024 - 1) / (fna2::kDecodeStages * fna2::decode_stage_bytes(a.head_dim, rc)));
+    const int64_t units = std::max<int64_t>((int64_t)a.batch * a.heads_kv, 1);
+    const double bytes = 2. * L * a.batch * (2. * a.heads_kv * a.head_dim +
+                                             (double)a.heads_graph * a.rank);
+    n = 1;
+    const double partials = 4. * a.batch * a.heads * a.head_dim;  // bytes a split
+    if (bytes >= (ragged ? kDecodeRagged : kDecodeLarge)) {
+      const int64_t fill = (int64_t)kDecodeCUs * std::min(per_cu, 4);
+      if (ragged) {
+        n = std::min(cdiv64(8 * fill, units), (int64_t)(0.006 * bytes / partials));
+        n = std::min(std::max<int64_t>(std::max(n, cdiv64(fill, units)), 4), cdiv64(steps, 8));
+      } else {
+        n = std::min(fill / units, cdiv64(steps, 4));
+      }
+      n = std::max<int64_t>(std::min<int64_t>(n, 64), 1);
+    } else {
+      // us; us a byte of the cache and of the partials
+      constexpr double kStart = 3.2, kMerge = 3.4, kRead = 0.16e-6, kPart = 0.8e-6;
+      const double step = 0.32 + 0.034 * rc + 0.38 * a.head_dim / 64;
+      const double cap = (double)kDecodeCUs * per_cu;
+      const double part = ragged ? 2. / 3 : 1.;  // of the longest
+      const double read = kRead * part * bytes;
+      double least = 0;
+      for (int64_t i = 1, last = 0; i <= std::min<int64_t>(steps, 64); ++i) {
+        const int64_t len = cdiv64(steps, i);  // steps a split
+        const int64_t count = cdiv64(steps, len);
+        if (count == last) continue;
+        last = count;
+        const double waves = (double)units * count;
+        auto round = [&](double w, double of) {
+          return std::max(kStart + of * len * step * (1 + 0.155 * std::max(w / kDecodeCUs - 1, 0.)),
+                          read * w / waves);
+        };
+        const double full = std::floor(waves / cap), rest = waves - full * cap;
+        double t = full > 0 ? full * round(cap, part) : 0;
+        if (rest > 0) t += round(rest, 1);
+        if (count > 1) t += kMerge + kPart * partials * count;
+        if (i == 1 || t < 0.98 * least) {
+          least = t;
+          n = count;
+        }
+      }
+    }
   }
-  n = std::min<int64_t>(n, cdiv64(L, 32));
+  n = std::min<int64_t>(n, steps);
   s.keys = (int)(cdiv64(cdiv64(L, n), 32) * 32);
   s.n = (int)cdiv64(L, s.keys);
   return s;

@@ -8,7 +8,7 @@ import torch
 from fna2_amd import _capi
 
 
-def _splits(B, H, HKV, HG, D, R, L):
+def _splits(B, H, HKV, HG, D, R, L, ragged=False):
     a = _capi.DecodeArgs()
     a.batch, a.heads, a.heads_kv, a.heads_graph = B, H, HKV, HG
     a.head_dim, a.rank, a.max_seqlen_k, a.softmax_scale = D, R, L, 0.1
@@ -16,12 +16,14 @@ def _splits(B, H, HKV, HG, D, R, L):
     for n in ("q", "r_q", "k_cache", "v_cache", "rk_cache", "out"):
         setattr(a, n, _capi.Tensor(fake, 1 << 20, 128, 1 << 14))
     a.graph_scale = fake
+    a.seqlens_k = fake if ragged else None
     return _capi.lib().fna2_decode_num_splits(ctypes.byref(a))
 
 
-@pytest.mark.parametrize("L,n", [(0, 1), (1, 1), (64, 1), (65, 3), (96, 3), (97, 4), (2048, 64),
+@pytest.mark.parametrize("L,n", [(0, 1), (1, 1), (64, 1), (65, 1), (128, 1), (160, 5), (2048, 64),
                                  (4096, 64)])
 def test_few_units_split_to_single_steps(L, n):
+    """Once the chain of steps is longer than a second launch."""
     assert _splits(1, 8, 8, 0, 128, 0, L) == n
 
 
@@ -29,7 +31,31 @@ def test_many_units_keep_long_splits():
     assert _splits(64, 16, 16, 16, 128, 32, 4096) == 1
     assert _splits(16, 16, 16, 16, 128, 32, 2048) == 4
     assert _splits(64, 16, 16, 16, 128, 32, 128) == 1
-    assert _splits(8, 32, 8, 0, 128, 0, 1024) == 8
+
+
+@pytest.mark.parametrize("call,most", [
+    # a few steps: a second launch costs more (measured whole / split, us)
+    ((4, 4, 1, 0, 64, 0, 84, True), 1),         # 5.2 / 7.4
+    ((87, 4, 1, 0, 64, 0, 84, True), 1),        # 5.6 / 7.9
+    ((2, 8, 2, 8, 128, 16, 73, True), 1),       # 8.0 / 9.9
+    ((13, 16, 16, 16, 64, 8, 116, True), 1),    # 7.9 / 9.1
+    ((97, 32, 32, 0, 128, 0, 304, True), 1),    # 59 / 72 to 123
+    # one round of the waves that fit, not a little more than one
+    ((118, 4, 2, 4, 128, 8, 305, False), 4),    # 15.1 in four, 19.2 in five
+    ((26, 32, 4, 32, 64, 16, 339, False), 6),   # 13.3 in six, 18.6 in eleven
+    ((1, 32, 32, 32, 128, 32, 1239, False), 20),  # 11.3 in twenty, 15.6 in 39
+    ((20, 32, 8, 0, 128, 0, 6000, False), 6),   # 90 in six, 104 in seven
+])
+def test_calls_not_split_further(call, most):
+    assert 1 <= _splits(*call) <= most
+
+
+@pytest.mark.parametrize("L", list(range(1, 400, 7)) + [1023, 4095, 131072, 2 ** 30])
+@pytest.mark.parametrize("B,H,HKV,HG,D,R", [(1, 1, 1, 0, 64, 0), (3, 32, 1, 8, 64, 32),
+                                            (300, 8, 8, 8, 128, 64), (2 ** 16, 32, 32, 0, 128, 0)])
+def test_counts_are_in_range(B, H, HKV, HG, D, R, L):
+    for ragged in (False, True):
+        assert 1 <= _splits(B, H, HKV, HG, D, R, L, ragged) <= min(64, -(-L // 32))
 
 
 def _one_step(a, b, absolute):
