@@ -370,82 +370,98 @@ __global__ __launch_bounds__(64 * kRopeWaves, kBwdOcc) void rope_norm_bwd_kernel
     const bool inside = p >= 0;
     float c[EPL], s[EPL];
     if (inside) tab.at(p, P.sign, lane, half, col, c, s);
-    // The q rows, then the k rows: one side's weights and pointers at a time.
-    static_for<2>([&](auto side_) {
-      constexpr int side = decltype(side_)::value;
-      const int rows = side ? P.Hk : P.Hq;
-      const bool has_w = (side ? P.wk : P.wq) != nullptr;
-      const char* xs = (const char*)(side ? P.k : P.q) + (int64_t)t * (side ? P.k_ss : P.q_ss) * ES;
-      const char* gs = (const char*)(side ? P.gk : P.gq) + (int64_t)t * (side ? P.gk_ss : P.gq_ss) * ES;
-      char* os = (char*)(side ? P.k_out : P.q_out) + (int64_t)t * (side ? P.ko_ss : P.qo_ss) * ES;
-      const int64_t xh = (side ? P.k_sh : P.q_sh) * ES, gh = (side ? P.gk_sh : P.gq_sh) * ES;
-      const int64_t oh = (side ? P.ko_sh : P.qo_sh) * ES;
-      for (int r0 = L.lrow; r0 - L.lrow < rows; r0 += NP * L.rpw) {
-        // every load of NP row passes first, as raw words
-        Raw<DT> x1[NP], x2[NP], g1[NP], g2[NP];
-#pragma unroll
-        for (int j = 0; j < NP; ++j) {
-          const int r = r0 + j * L.rpw;
-          x1[j].w = x2[j].w = g1[j].w = g2[j].w = u32x4{0u, 0u, 0u, 0u};
-          if (r < rows) {
-            x1[j].load(xs + r * xh + col * ES);
-            x2[j].load(xs + r * xh + (half + col) * ES);
-            g1[j].load(gs + r * gh + col * ES);
-            g2[j].load(gs + r * gh + (half + col) * ES);
-          }
+    // Up to two row passes at once: slot j takes row `r` of side `side`
+    // (0: q, 1: k), a compile-time one: its weights and pointers.
+    auto passes = [&](auto n_, auto side0_, auto side1_, int row0, int row1) {
+      constexpr int N = decltype(n_)::value;
+      // every load first, as raw words
+      Raw<DT> x1[N], x2[N], g1[N], g2[N];
+      static_for<N>([&](auto j_) {
+        constexpr int j = decltype(j_)::value;
+        constexpr int side = j ? decltype(side1_)::value : decltype(side0_)::value;
+        const int r = j ? row1 : row0;
+        x1[j].w = x2[j].w = g1[j].w = g2[j].w = u32x4{0u, 0u, 0u, 0u};
+        if (r < (side ? P.Hk : P.Hq)) {
+          const char* xs = (const char*)(side ? P.k : P.q) + (int64_t)t * (side ? P.k_ss : P.q_ss) * ES;
+          const char* gs = (const char*)(side ? P.gk : P.gq) + (int64_t)t * (side ? P.gk_ss : P.gq_ss) * ES;
+          const char* x = xs + r * ((side ? P.k_sh : P.q_sh) * ES);
+          const char* g = gs + r * ((side ? P.gk_sh : P.gq_sh) * ES);
+          x1[j].load(x + col * ES);
+          x2[j].load(x + (half + col) * ES);
+          g1[j].load(g + col * ES);
+          g2[j].load(g + (half + col) * ES);
         }
-#pragma unroll
-        for (int j = 0; j < NP; ++j) {
-          const int r = r0 + j * L.rpw;
-          const bool live = r < rows;
-          if (!inside) {  // (the same for every lane)
-            if (live) {
-              g1[j].store(os + r * oh + col * ES);
-              g2[j].store(os + r * oh + (half + col) * ES);
-            }
-            continue;
-          }
-          // g' = R(-angle) dy (the transpose of the forward rotation)
-          Ch y1, y2;
-          float ss = 0.f, tw = 0.f;
-#pragma unroll
-          for (int e = 0; e < EPL; ++e) {
-            const float a = g1[j].get(e), b = g2[j].get(e);
-            const float u = x1[j].get(e), v = x2[j].get(e);
-            y1.v[e] = add_rn(mul_rn(a, c[e]), mul_rn(b, s[e]));
-            y2.v[e] = add_rn(mul_rn(b, c[e]), mul_rn(-a, s[e]));
-            ss += u * u + v * v;
-            tw += u * wsh[side][col + e] * y1.v[e] + v * wsh[side][half + col + e] * y2.v[e];
-          }
-          // (a lane past the rows holds zeros; every lane joins the sums)
-          ss = row_sum(ss, L.lpr);
-          tw = row_sum(tw, L.lpr);
-          // (fp16: the products below stay behind the sums.  Begun ahead of
-          // them, they spilled 9 registers: 16384 tokens, d128 91.0 -> 90.1
-          // us, 6000 35.2 -> 34.5, 3000 26.5 -> 26.8.  In bf16 they spill
-          // one, outside the loop; there the order costs 1 to 3%.)
-          if constexpr (DT == kRopeF16) asm volatile("" : "+v"(ss));
-          if (has_w) {
-            const float rr = rsqrtf(ss * inv_d + P.eps);
-            const float k3 = rr * rr * rr * tw * inv_d;
-            if (live) {
-#pragma unroll
-              for (int e = 0; e < EPL; ++e) {
-                const float u = x1[j].get(e), v = x2[j].get(e);
-                dw1[side][e] += u * rr * y1.v[e];
-                dw2[side][e] += v * rr * y2.v[e];
-                y1.v[e] = rr * wsh[side][col + e] * y1.v[e] - u * k3;
-                y2.v[e] = rr * wsh[side][half + col + e] * y2.v[e] - v * k3;
-              }
-            }
-          }
+      });
+      static_for<N>([&](auto j_) {
+        constexpr int j = decltype(j_)::value;
+        constexpr int side = j ? decltype(side1_)::value : decltype(side0_)::value;
+        const int r = j ? row1 : row0;
+        const bool live = r < (side ? P.Hk : P.Hq);
+        char* os = (char*)(side ? P.k_out : P.q_out) + (int64_t)t * (side ? P.ko_ss : P.qo_ss) * ES;
+        const int64_t oh = (side ? P.ko_sh : P.qo_sh) * ES;
+        if (!inside) {  // (the same for every lane)
           if (live) {
-            y1.store(os + r * oh + col * ES);
-            y2.store(os + r * oh + (half + col) * ES);
+            g1[j].store(os + r * oh + col * ES);
+            g2[j].store(os + r * oh + (half + col) * ES);
+          }
+          return;
+        }
+        // g' = R(-angle) dy (the transpose of the forward rotation)
+        Ch y1, y2;
+        float ss = 0.f, tw = 0.f;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+          const float a = g1[j].get(e), b = g2[j].get(e);
+          const float u = x1[j].get(e), v = x2[j].get(e);
+          y1.v[e] = add_rn(mul_rn(a, c[e]), mul_rn(b, s[e]));
+          y2.v[e] = add_rn(mul_rn(b, c[e]), mul_rn(-a, s[e]));
+          ss += u * u + v * v;
+          tw += u * wsh[side][col + e] * y1.v[e] + v * wsh[side][half + col + e] * y2.v[e];
+        }
+        // (a lane past the rows holds zeros; every lane joins the sums)
+        ss = row_sum(ss, L.lpr);
+        tw = row_sum(tw, L.lpr);
+        // (fp16: the products below stay behind the sums.  Begun ahead of
+        // them, they spilled 9 registers: 16384 tokens, d128 91.0 -> 90.1
+        // us, 6000 35.2 -> 34.5, 3000 26.5 -> 26.8.  In bf16 the order
+        // costs 1 to 3%.)
+        if constexpr (DT == kRopeF16) asm volatile("" : "+v"(ss));
+        if ((side ? P.wk : P.wq) != nullptr) {
+          const float rr = rsqrtf(ss * inv_d + P.eps);
+          const float k3 = rr * rr * rr * tw * inv_d;
+          if (live) {
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) {
+              const float u = x1[j].get(e), v = x2[j].get(e);
+              dw1[side][e] += u * rr * y1.v[e];
+              dw2[side][e] += v * rr * y2.v[e];
+              y1.v[e] = rr * wsh[side][col + e] * y1.v[e] - u * k3;
+              y2.v[e] = rr * wsh[side][half + col + e] * y2.v[e] - v * k3;
+            }
           }
         }
-      }
-    });
+        if (live) {
+          y1.store(os + r * oh + col * ES);
+          y2.store(os + r * oh + (half + col) * ES);
+        }
+      });
+    };
+    constexpr std::integral_constant<int, NP> np{};
+    constexpr std::integral_constant<int, 0> q_{};
+    constexpr std::integral_constant<int, 1> k_{};
+    const int q0 = L.lrow;
+    bool together = false;
+    if constexpr (NP == 2) together = max(P.Hq, P.Hk) <= L.rpw;
+    if (together) {
+      // A pass has room for all of a side's rows: both sides' together, so
+      // that the token waits for its loads once (fp32, 40000 tokens: d64 1/1
+      // heads 55 us, one after the other 70; d128 4/2 89, 105).  Not with
+      // more rows: d64 16/4 at 15000 tokens 49.9, one after the other 48.4.
+      if constexpr (NP == 2) passes(np, q_, k_, q0, q0);
+    } else {
+      for (int r = q0; r - q0 < P.Hq; r += NP * L.rpw) passes(np, q_, q_, r, r + L.rpw);
+      for (int r = q0; r - q0 < P.Hk; r += NP * L.rpw) passes(np, k_, k_, r, r + L.rpw);
+    }
   }
 
   // dw partials: lanes sharing columns (lane % lpr), then the waves, in a

@@ -30,6 +30,8 @@ CASES = [  # T, Hq, Hk, D
     (1, 1, 1, 64), (3, 3, 1, 128), (1024, 5, 2, 128), (1025, 4, 4, 64), (4096, 3, 3, 128),
     (4097, 2, 1, 128), (12288, 2, 2, 64), (12289, 1, 3, 64), (37, 9, 17, 16), (50, 2, 2, 512),
     (130, 0, 4, 256),
+    # fp32, q and k in one pass: as many rows as it has, one more, one side empty
+    (200, 8, 8, 64), (201, 9, 1, 64), (90, 4, 4, 128), (91, 1, 5, 128), (70, 1, 1, 512), (40, 0, 3, 128),
 ]
 
 
