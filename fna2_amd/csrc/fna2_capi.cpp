@@ -245,6 +245,10 @@ int dq_groups(const fna2_problem& p) {
 // of those that cost a pack of its mean length nothing: up to 1.1 times the
 // whole items by this estimate, in 2 to 8 chunks (of 33 such packs measured
 // none was slower; of 27 between 1.2 and 1.4, 12 were, and 16 chunks at 1.1).
+// A max_seqlen that is the token count names no length, so whole items of it
+// make no rounds that chunks would shorten ([8000, 900, 700, 617], H32/8 d128
+// r64, not causal: 4.81 ms whole, 5.09 in halves; of 20 such packs 18 were 1
+// to 13% slower in chunks; with a true or no max_seqlen 3 of 11).
 //
 // Measured (dK/dV and its reduction, us, whole items -> the rule's chunks):
 // B2 H16/4 L1531 d128 fp16 238 -> 88 (chunks of 1/2: 138, 1/4: 86, 1/8: 96,
@@ -286,13 +290,13 @@ KvSplit kv_split(const fna2_problem& p) {
     return w;
   };
   constexpr double kEnter = 4, kLaunch = 5, kBytesPerBlock = 4e6;
-  auto cost = [&](const Work& w, int log2) {
+  auto cost = [&](const Work& w, int log2, bool rounds) {
     const int64_t n = (int64_t)1 << log2;
     const int64_t len = std::max<int64_t>(cdiv64(w.longest, n), log2 ? fna2::kKvMinChunk : 1);
     const double chunks = std::min((double)w.items * n,
                                    std::max((double)w.total / fna2::kKvMinChunk, (double)w.items));
     double t = std::max(len + kEnter, (w.total + kEnter * chunks) / kSplitCUs);
-    if (!p.causal)
+    if (rounds)
       t = std::max(t, cdiv64(w.items * cdiv64(w.longest, len), kSplitCUs) * (len + kEnter));
     if (log2 > 0) t += kLaunch + chunks * bn * (2 * p.head_dim + rpl) * 8.0 / kBytesPerBlock;
     return t;
@@ -310,8 +314,10 @@ KvSplit kv_split(const fna2_problem& p) {
   // lengths every tile is cut, in others the shortest may stay whole)
   const int64_t cut =
       std::min(g.kv_tiles, std::max(p.batch * even.kt, p.varlen ? cdiv64(p.total_k, bn) + 8 : 0));
-  double least = 0.9 * cost(hinted, 0);
-  const double whole = cost(even, 0);
+  const bool alike = !p.causal;  // (`rounds`: see above)
+  const bool told = alike && !(p.varlen && p.batch > 1 && p.seqlen_k >= p.total_k);
+  double least = 0.9 * cost(hinted, 0, told);
+  const double whole = cost(even, 0, alike);
   for (int log2 = 1; log2 <= 4; ++log2) {
     KvSplit s;
     s.log2 = log2;
@@ -324,8 +330,8 @@ KvSplit kv_split(const fna2_problem& p) {
     if (s.tiles <= 0 || (s.tiles * p.heads_kv) << log2 > kMaxGrid) continue;
     s.drk_part = align_up((size_t)(s.tiles * kv));
     s.bytes = s.drk_part + align_up((size_t)(s.tiles * dr));
-    if (cost(even, log2) > (log2 < 4 && hinted.longest > even.longest ? 1.1 : 0.9) * whole) continue;
-    const double t = cost(hinted, log2);
+    if (cost(even, log2, alike) > (log2 < 4 && hinted.longest > even.longest ? 1.1 : 0.9) * whole) continue;
+    const double t = cost(hinted, log2, alike);
     if (t < least) {
       least = t;
       best = s;

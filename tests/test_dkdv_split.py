@@ -273,3 +273,19 @@ def test_equal_chunks_go_in_whole_rounds():
     # 104 items: one round of halves
     halves = 2 * 13 * 4 * 256 * 4 * ((2 * 64 << 1) + (3 + (1 << 1) - 1) * 32)
     assert _split_bytes(_problem(False, 2, 3209, 3209, 12, 4, 12, 64, 16, False)) == halves
+
+
+def test_token_count_as_max_seqlen_makes_no_rounds():
+    """Lengths of 8000, 900, 700 and 617: 504 long items that 256 CUs share,
+    not three rounds of them, whatever max_seqlen says; but one long sequence
+    whose items do leave CUs idle is cut, and so is a pack of one sequence,
+    whose items are alike."""
+    def pack(total, n, hint, H, HKV, D, R):
+        p = _problem(True, n, hint, hint, H, HKV, H if R else 0, D, R, False, None)
+        p.total_q = p.total_k = total
+        p.cu_seqlens_q = p.cu_seqlens_k = 1 << 20
+        return _split_bytes(p)
+    for hint in (0, 8000, 10217):
+        assert pack(10217, 4, hint, 32, 8, 128, 64) == 0
+    assert pack(10533, 4, 7083, 12, 4, 64, 0) > 0
+    assert pack(4824, 1, 4824, 16, 8, 128, 16) > 0
