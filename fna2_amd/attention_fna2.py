@@ -733,25 +733,26 @@ class NaylisAttention(nn.Module):
                 type(cache) is not StaticKVCache or n >= cache.capacity or
                 (cache.r_k is None) != (r_k is None) or nn.modules.module._has_any_global_hook()):
             return None
-        for m, cls in ((self.q_norm, RMSNorm), (self.k_norm, RMSNorm),
-                       (self.rope, RotaryPositionalEmbedding)):
+        qn, kn, rope = self.q_norm, self.k_norm, self.rope
+        for m, cls in ((qn, RMSNorm), (kn, RMSNorm), (rope, RotaryPositionalEmbedding)):
             if m is not None and (type(m) is not cls or m._forward_hooks or
                                   m._forward_pre_hooks or "forward" in vars(m)):
                 return None  # a replaced or hooked module is called as such
+        wq, wk = None if qn is None else qn.weight, None if kn is None else kn.weight
         nat = _capi.native_or_none() if q.is_cuda else None
-        if nat is None or any(t.dtype != torch.bfloat16 for t in (
-                q, *(m.weight for m in (self.q_norm, self.k_norm) if m is not None))):
+        if nat is None or q.dtype != torch.bfloat16 or any(
+                w is not None and w.dtype != torch.bfloat16 for w in (wq, wk)):
             return None  # (the modules' table is then of another dtype: see _table)
         cos = sin = None
-        if self.rope is not None:
-            cos, sin = self.rope._table(n + 1, q.device, q.dtype)
+        if rope is not None:
+            cos, sin = rope._table(n + 1, q.device, q.dtype)
             cos, sin = cos[n], sin[n]
         norm = self.use_qk_norm
         out = nat.decode_rows(
             q, k, v, r_k, cache.k[:, :, n:n + 1], cache.v[:, :, n:n + 1],
             None if r_k is None else cache.r_k[:, :, n:n + 1],
-            self.q_norm.weight if norm else None, self.q_norm.eps if norm else 0.0,
-            self.k_norm.weight if norm else None, self.k_norm.eps if norm else 0.0, cos, sin)
+            wq if norm else None, qn.eps if norm else 0.0,
+            wk if norm else None, kn.eps if norm else 0.0, cos, sin)
         if out is None:
             return None
         cache.length = n + 1

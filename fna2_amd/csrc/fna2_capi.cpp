@@ -1188,8 +1188,8 @@ int fna2_check_decode(const fna2_decode_args* a) {
     if ((gg - 1) * a->rk_cache.stride_h * 2 + 31 * a->rk_cache.stride_s * 2 + R * 2 > kOff31)
       return FNA2_E_SHAPE;
   }
-  const DecSplit s = dec_split(*a);
-  if ((int64_t)a->batch * a->heads_kv * s.n > kMaxGrid) return FNA2_E_SHAPE;
+  const int64_t units = (int64_t)a->batch * a->heads_kv;  // (at most 64 splits)
+  if (units > kMaxGrid / 64 && units * dec_split(*a).n > kMaxGrid) return FNA2_E_SHAPE;
   return FNA2_OK;
 }
 
